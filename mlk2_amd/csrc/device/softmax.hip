@@ -12,6 +12,8 @@
 // no barriers. exp runs in f32 on x - r (x - r is exact whenever x is near r,
 // which is where the large outputs are); the row sum accumulates in f64, so
 // the normalisation error stays ~1 f32 ULP of each output.
+// Longer f32 rows and f16 rows (16 to 65536 columns): softmaxRowWide, the row
+// in registers, f64 arithmetic.
 // General path (any dtype, any cols): one workgroup per row, three passes over
 // the row with LDS reductions, f64 throughout.
 #include <hip/hip_runtime.h>
@@ -39,6 +41,10 @@ __device__ __forceinline__ double waveSum(double v) {
     for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
     return v;
 }
+
+/// Waves a row of softmaxWaveRowScalar<CH> is split over.
+template <int CH>
+constexpr int kScalarWaves = CH > 16 ? 4 : 1;
 
 /// Loads one row into the lane's CH float4 (columns past `cols` read as -inf,
 /// which leaves the max unchanged and adds exp(-inf) = 0 to nothing: the sum
@@ -137,45 +143,77 @@ __global__ __launch_bounds__(256) void softmaxWaveRow(const float* x,
     }
 }
 
+/// A workgroup barrier that orders LDS alone: __syncthreads would also wait
+/// for every global load and store in flight.
+__device__ __forceinline__ void ldsBarrier() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
+    __builtin_amdgcn_s_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
+}
+
+/// Max (MAX) or sum of one value per wave over the W waves of a row, in every
+/// lane. `slot` is the row's LDS array; a row's max and sum use two arrays, so
+/// the barrier of one separates the reads of the other from its next writes.
+template <int W, bool MAX, typename T>
+__device__ __forceinline__ T acrossWaves(T v, T (&slot)[W]) {
+    if constexpr (W > 1) {
+        if ((threadIdx.x & 63) == 0) slot[threadIdx.x >> 6] = v;
+        ldsBarrier();
+        v = slot[0];
+#pragma unroll
+        for (int i = 1; i < W; ++i) {
+            if constexpr (MAX) v = fmaxf(v, slot[i]);
+            else v += slot[i];
+        }
+    }
+    return v;
+}
+
 /// Rows the float4 loads cannot take (cols % 4 != 0, or a row start off 16
-/// bytes), up to 256 * CH columns: one wave per row with the arithmetic of
-/// softmaxWaveRow<CH, true, true> (f32 max, v_exp_f32, f64 sum of f32 sums
-/// of 4-element groups), 4-byte loads and stores that are lane-contiguous
-/// per instruction. v[c][e] holds element c * 256 + e * 64 + lane; elements
-/// past the row read as -inf and add exp2(-inf) = 0 to their group.
+/// bytes), up to 256 * CH columns: the arithmetic of softmaxWaveRow<CH, true,
+/// true> (f32 max, v_exp_f32, f64 sum of f32 sums of 4-element groups), 4-byte
+/// loads and stores that are lane-contiguous per instruction. One wave per row
+/// up to 4096 columns; past that the row is split over 4 waves, since one wave
+/// would hold 128 row registers beside their addresses and spill. v[c][e]
+/// holds element (c * W + wave) * 256 + e * 64 + lane; elements past the row
+/// read as -inf and add exp2(-inf) = 0 to their group.
 template <int CH>
 __global__ __launch_bounds__(256) void softmaxWaveRowScalar(const float* __restrict__ x, float* __restrict__ y,
                                                             int64_t rows, int64_t cols, int64_t xs, int64_t ys) {
+    constexpr int W = kScalarWaves<CH>, N = CH / W;
+    __shared__ float smax[W];
+    __shared__ double ssum[W];
     const int lane = threadIdx.x & 63;
-    const int64_t wave = static_cast<int64_t>(blockIdx.x) * 4 + (threadIdx.x >> 6);
-    const int64_t waves = static_cast<int64_t>(gridDim.x) * 4;
-    for (int64_t row = wave; row < rows; row += waves) {
+    const int w = W > 1 ? threadIdx.x >> 6 : 0;
+    const int64_t rowsPer = 4 / W;
+    const int64_t first = static_cast<int64_t>(blockIdx.x) * rowsPer + (W > 1 ? 0 : threadIdx.x >> 6);
+    for (int64_t row = first; row < rows; row += static_cast<int64_t>(gridDim.x) * rowsPer) {
         const float* xr = x + row * xs;
         float* yr = y + row * ys;
-        f32x4 v[CH];
+        f32x4 v[N];
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
+        for (int c = 0; c < N; ++c) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int64_t col = static_cast<int64_t>(c) * 256 + e * 64 + lane;
+                const int64_t col = static_cast<int64_t>(c * W + w) * 256 + e * 64 + lane;
                 v[c][e] = col < cols ? xr[col] : -INFINITY;
             }
         }
-        const float m = rowMax<CH>(v);
+        const float m = acrossWaves<W, true>(rowMax<N>(v), smax);
         double s = 0.0;
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
+        for (int c = 0; c < N; ++c) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) v[c][e] = __builtin_amdgcn_exp2f((v[c][e] - m) * 1.44269504088896340736f);
             s += static_cast<double>((v[c][0] + v[c][1]) + (v[c][2] + v[c][3]));
         }
-        s = waveSum(s);
+        s = acrossWaves<W, false>(waveSum(s), ssum);
         const float inv = static_cast<float>(1.0 / s);
 #pragma unroll
-        for (int c = 0; c < CH; ++c) {
+        for (int c = 0; c < N; ++c) {
 #pragma unroll
             for (int e = 0; e < 4; ++e) {
-                const int64_t col = static_cast<int64_t>(c) * 256 + e * 64 + lane;
+                const int64_t col = static_cast<int64_t>(c * W + w) * 256 + e * 64 + lane;
                 if (col < cols) __builtin_nontemporal_store(v[c][e] * inv, yr + col);
             }
         }
@@ -236,6 +274,209 @@ __global__ __launch_bounds__(256) void softmaxWaveRowPipelined(const float* x, f
         finishRow<CH, false, true, false>(cur, y + row * ys, cols, lane);
 #pragma unroll
         for (int c = 0; c < CH; ++c) cur[c] = nxt[c];
+    }
+}
+
+/// 2^f on |f| <= 1/2 by Chebyshev interpolation at N nodes: relative error
+/// 2.5e-9 (N = 7), 5.5e-11 (N = 8), 1.9e-14 (N = 10).
+constexpr double kExp2C7[7] = {1.0,
+                               0.6931472067028326,
+                               0.24022650922288757,
+                               0.05550327226670302,
+                               0.009618056678524643,
+                               0.0013400428177615916,
+                               0.00015461444698568514};
+constexpr double kExp2C8[8] = {0.9999999999595618,     0.6931471805568324,    0.24022651213498092,
+                               0.055504109063258665,   0.009618025613318018,  0.0013333478473685175,
+                               0.00015469729214122798, 1.5303700711425663e-05};
+constexpr double kExp2C10[10] = {1.0000000000000135,    0.6931471805599462,     0.2402265069564034,
+                                 0.05550410866465166,   0.00961812919393429,    0.0013333558200796013,
+                                 0.0001540343375126647, 1.5252672924257465e-05, 1.3259645241948732e-06,
+                                 1.020590550210069e-07};
+
+/// 2^y (times the coefficients' common factor) for y in [-1000, 1000]; NaN
+/// stays NaN. y + 1.5 * 2^52 leaves rint(y) in the low word, from where it is
+/// added into the exponent field.
+template <int N>
+__device__ __forceinline__ double exp2Poly(double y, const double (&c)[N]) {
+    const double t = y + 0x1.8p52;
+    const double f = y - (t - 0x1.8p52);
+    double p = c[N - 1];
+#pragma unroll
+    for (int i = N - 2; i >= 0; --i) p = __builtin_fma(p, f, c[i]);
+    return __hiloint2double(__double2hiint(p) + (__double2loint(t) << 20), __double2loint(p));
+}
+
+template <typename T>
+struct WideRow;
+template <>
+struct WideRow<float> {
+    static constexpr int V = 4;
+    static constexpr float kMostMax = 1e6f;
+    using Vec = f32x4;
+    static constexpr const auto& cSum = kExp2C7;
+    static constexpr const auto& cOut = kExp2C8;
+    static __device__ __forceinline__ float narrow(double v) { return static_cast<float>(v); }
+};
+template <>
+struct WideRow<_Float16> {
+    static constexpr int V = 8;
+    static constexpr float kMostMax = 60000.0f;
+    using Vec = _Float16 __attribute__((ext_vector_type(8)));
+    static constexpr const auto& cSum = kExp2C10;
+    static constexpr const auto& cOut = kExp2C10;
+    /// One rounding of v >= 0: to the nearest f32, made round-to-odd (one
+    /// step down if that was up, the last bit set if inexact), then to f16.
+    static __device__ __forceinline__ _Float16 narrow(double v) {
+        const float r = static_cast<float>(v);
+        const double d = static_cast<double>(r);
+        uint32_t bits = __float_as_uint(r) - (d > v ? 1u : 0u);
+        bits |= d != v ? 1u : 0u;
+        return static_cast<_Float16>(__uint_as_float(bits));
+    }
+};
+
+/// softmaxRowWide's row for a max that is infinite or so large that floats
+/// near it lie far apart (or, in f16, end): the same arithmetic, element by
+/// element from memory, with the exponent itself held at -1000 or more. x and
+/// y may be the same row: each element is read before its thread writes it.
+template <typename T, int W>
+__device__ __forceinline__ void softmaxOddRow(const T* x, T* y, int cols, float m, int thread, double (&slot)[W]) {
+    using R = WideRow<T>;
+    const double mb = static_cast<double>(m) * -1.4426950408889634074;
+    auto term = [&](T xv) {
+        const double e = __builtin_fma(static_cast<double>(static_cast<float>(xv)), 1.4426950408889634074, mb);
+        return exp2Poly(e < -1000.0 ? -1000.0 : e, kExp2C10);
+    };
+    double s = 0.0;
+#pragma unroll 1
+    for (int i = thread; i < cols; i += 64 * W) s += term(x[i]);
+    s = acrossWaves<W, false>(waveSum(s), slot);
+    const double inv = 1.0 / s;
+#pragma unroll 1
+    for (int i = thread; i < cols; i += 64 * W) y[i] = R::narrow(term(x[i]) * inv);
+}
+
+/// Rows past the float4 path's 8192 columns and rows of f16, in f64
+/// arithmetic with one rounding to T (the general kernel's precision): W waves
+/// per row, CH 16-byte pieces of it in each lane's registers in T, so the row
+/// is read once and written once. Pieces start at the row's first 16-byte
+/// boundary; the up to V - 1 elements before it and after the last whole
+/// piece go one to a lane of the first wave. 2^y takes 12-15 f64 instructions
+/// (which issue at the f32 rate here), so it is computed twice, for the sum
+/// and for the output, rather than held in two registers per element.
+/// 1000 x 30001 f32 takes 57 us, 4.2 TB/s (softmaxBlockRow, which reads the row
+/// three times and calls exp twice: 219 us; a copy of the same bytes: 45 us),
+/// 8192 x 4096 f16 54 us (160 us). The f64 work, about 30 us of each, and the
+/// memory traffic overlap only between the two to four rows a CU holds.
+/// Summing against a reference of the row's first pieces, so that a piece's
+/// terms are computed under the loads of the next, took 72 us; walking rows
+/// with the next one's loads in flight 60 us (both need more registers).
+template <typename T, int CH, int W>
+__global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softmaxRowWide(const T* x, T* y, int64_t rows, int cols,
+                                                                           int64_t stride) {
+    using R = WideRow<T>;
+    using Vec = typename R::Vec;
+    constexpr int V = R::V;
+    constexpr int NOut = sizeof(R::cOut) / sizeof(double);
+    __shared__ float smax[W];
+    __shared__ double ssum[W];
+    const int lane = threadIdx.x & 63;
+    const int w = W > 1 ? threadIdx.x >> 6 : 0;
+    const int piece = w * 64 + lane;
+    const int64_t row = W > 1 ? static_cast<int64_t>(blockIdx.x)
+                              : static_cast<int64_t>(blockIdx.x) * 4 +
+                                    __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    if (row >= rows) return;
+    const T* xr = x + row * stride;
+    T* yr = y + row * stride;
+    // The row's first boundary, whole pieces (one or more), and this lane's
+    // single element (-1: none).
+    const int head = static_cast<int>((-reinterpret_cast<uintptr_t>(xr) & 15) / sizeof(T));
+    const int whole = (cols - head) / V;
+    const int tail = cols - head - whole * V;
+    const int single = piece < head ? piece : (piece < head + tail ? cols - tail + (piece - head) : -1);
+    const T kNone = static_cast<T>(-INFINITY);
+    T one = kNone;
+    if (single >= 0) one = xr[single];
+    // A piece past the row is the row's last one again, set to -inf below:
+    // with no branch around the loads, the wait for one leaves those behind it
+    // in flight.
+    Vec v[CH];
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        const int first = c * (W * 64);
+        const uint32_t off = static_cast<uint32_t>(min(piece, whole - 1 - first) + first) * 16u;
+        v[c] = *reinterpret_cast<const Vec*>(reinterpret_cast<const char*>(xr + head) + off);
+    }
+    float m = static_cast<float>(one);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        if (whole < (c + 1) * (W * 64)) {
+            const bool in = piece < whole - c * (W * 64);
+#pragma unroll
+            for (int i = 0; i < V; ++i) v[c][i] = in ? v[c][i] : kNone;
+        }
+#pragma unroll
+        for (int i = 0; i < V; ++i) m = fmaxf(m, static_cast<float>(v[c][i]));
+    }
+    m = acrossWaves<W, true>(waveMax(m), smax);
+    // exp(x - m) = 2^(x log2(e) - m log2(e)). Elements more than 300 below
+    // the max (and the -inf of elements past the row) become m - 300, whose
+    // result rounds to the same zero; NaN stays NaN. Where m - 300 is no value
+    // of T near it, or m is infinite, softmaxOddRow runs.
+    if (!(fabsf(m) <= R::kMostMax)) {
+        softmaxOddRow<T, W>(xr, yr, cols, m, piece, ssum);
+        return;
+    }
+    const T lo = static_cast<T>(m - 300.0f);
+    const double mb = static_cast<double>(m) * -1.4426950408889634074;
+    auto exponent = [&](T xv) {
+        return __builtin_fma(static_cast<double>(static_cast<float>(xv)), 1.4426950408889634074, mb);
+    };
+    double s = 0.0;
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+#pragma unroll
+        for (int i = 0; i < V; ++i) {
+            v[c][i] = v[c][i] < lo ? lo : v[c][i];
+            s += exp2Poly(exponent(v[c][i]), R::cSum);
+        }
+        // The terms are recomputed below, not kept.
+        asm volatile("" : "+v"(v[c]), "+v"(s));
+    }
+    if (w == 0) {
+        one = one < lo ? lo : one;
+        s += exp2Poly(exponent(one), R::cSum);
+    }
+    s = acrossWaves<W, false>(waveSum(s), ssum);
+    // s >= 1 or NaN, as in normalizeRow. A NaN row's outputs are all NaN (set
+    // at the end: the exponent add would spoil a NaN coefficient).
+    const bool bad = !(s > 0.0);
+    const double inv = bad ? 0.0 : 1.0 / s;
+    double co[NOut];
+#pragma unroll
+    for (int i = 0; i < NOut; ++i) {   // uniform over the row's waves: scalar registers
+        const double k = R::cOut[i] * inv;
+        co[i] = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(k)),
+                                 __builtin_amdgcn_readfirstlane(__double2loint(k)));
+    }
+    const float nan = static_cast<float>(s);
+    auto result = [&](T xv) {
+        const T r = R::narrow(exp2Poly(exponent(xv), co));
+        return bad ? static_cast<T>(nan) : r;
+    };
+    if (single >= 0) yr[single] = result(one);
+#pragma unroll
+    for (int c = 0; c < CH; ++c) {
+        Vec o;
+#pragma unroll
+        for (int i = 0; i < V; ++i) o[i] = result(v[c][i]);
+        const int first = c * (W * 64);
+        char* base = reinterpret_cast<char*>(yr + head) + first * 16;
+        if (piece < whole - first) {
+            __builtin_nontemporal_store(o, reinterpret_cast<Vec*>(base + static_cast<uint32_t>(piece) * 16u));
+        }
     }
 }
 
@@ -348,12 +589,71 @@ int launchWave(const mlkd_softmax& p, hipStream_t st) {
 
 template <int CH>
 int launchScalar(const mlkd_softmax& p, hipStream_t st) {
-    int64_t blocks = (p.rows + 3) / 4;
+    constexpr int64_t rowsPer = 4 / kScalarWaves<CH>;
+    int64_t blocks = (p.rows + rowsPer - 1) / rowsPer;
     if (blocks > 8192) blocks = 8192;
     hipLaunchKernelGGL(softmaxWaveRowScalar<CH>, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st,
                        static_cast<const float*>(p.x), static_cast<float*>(p.y), p.rows, p.cols, p.x_row_stride,
                        p.y_row_stride);
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
+}
+
+/// softmaxRowWide applies to one dtype in and out (f32 or f16), rows of x and
+/// y with the same offset from a 16-byte boundary, 16 (a whole piece)
+/// to 65536 columns: what the registers of 16 waves hold.
+bool wideApplies(const mlkd_softmax* p) {
+    const bool f32 = p->x_dtype == MLKD_F32 && p->y_dtype == MLKD_F32;
+    const bool f16 = p->x_dtype == MLKD_F16 && p->y_dtype == MLKD_F16;
+    const int64_t es = f32 ? 4 : 2;
+    return (f32 || f16) && p->cols >= 16 && p->cols >= 16 && p->rows <= 0x7FFFFFFF && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->x_row_stride == p->y_row_stride && p->cols <= 65536 &&
+           ((reinterpret_cast<uintptr_t>(p->x) ^ reinterpret_cast<uintptr_t>(p->y)) & 15u) == 0 &&
+           reinterpret_cast<uintptr_t>(p->x) % static_cast<uintptr_t>(es) == 0;
+}
+
+template <typename T, int CH, int W>
+int launchWideAs(const mlkd_softmax& p, hipStream_t st) {
+    const int64_t blocks = W > 1 ? p.rows : (p.rows + 3) / 4;
+    hipLaunchKernelGGL((softmaxRowWide<T, CH, W>), dim3(static_cast<unsigned>(blocks)), dim3(W == 1 ? 256 : 64 * W), 0,
+                       st, static_cast<const T*>(p.x), static_cast<T*>(p.y), p.rows, static_cast<int>(p.cols),
+                       p.x_row_stride);
+    return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
+}
+
+/// Waves per row (w) and pieces per lane (ch) by row length. f16 rows up to
+/// 2048 columns take one wave and no barrier.
+struct WideShape {
+    int ch, w;
+};
+
+WideShape wideShape(const mlkd_softmax& p) {
+    if (p.x_dtype == MLKD_F16) {
+        const int64_t c = p.cols;
+        if (c <= 512) return {1, 1};
+        if (c <= 1024) return {2, 1};
+        if (c <= 2048) return {4, 1};
+        if (c <= 4096) return {2, 4};
+        if (c <= 8192) return {4, 4};
+        if (c <= 16384) return {4, 8};
+        return c <= 32768 ? WideShape{4, 16} : WideShape{8, 16};
+    }
+    const int64_t c = p.cols;
+    if (c <= 16384) return {16, 4};
+    return c <= 32768 ? WideShape{16, 8} : WideShape{16, 16};
+}
+
+int launchWide(const mlkd_softmax& p, hipStream_t st) {
+    const WideShape f = wideShape(p);
+    if (p.x_dtype == MLKD_F16) {
+        if (f.w == 1) {
+            if (f.ch == 1) return launchWideAs<_Float16, 1, 1>(p, st);
+            return f.ch == 2 ? launchWideAs<_Float16, 2, 1>(p, st) : launchWideAs<_Float16, 4, 1>(p, st);
+        }
+        if (f.w == 4) return f.ch == 2 ? launchWideAs<_Float16, 2, 4>(p, st) : launchWideAs<_Float16, 4, 4>(p, st);
+        if (f.w == 8) return launchWideAs<_Float16, 4, 8>(p, st);
+        return f.ch == 4 ? launchWideAs<_Float16, 4, 16>(p, st) : launchWideAs<_Float16, 8, 16>(p, st);
+    }
+    if (f.w == 4) return launchWideAs<float, 16, 4>(p, st);
+    return f.w == 8 ? launchWideAs<float, 16, 8>(p, st) : launchWideAs<float, 16, 16>(p, st);
 }
 
 /// f32 rows up to 8192 columns that the float4 path does not take.
@@ -377,7 +677,13 @@ extern "C" const char* mlkd_softmax_kernel_name(const mlkd_softmax* p) {
     int ch = 1;
     while (256 * ch < p->cols) ch *= 2;
     if (!(p->x_dtype == MLKD_F32 && p->y_dtype == MLKD_F32 && (p->cols & 3) == 0 && aligned && p->cols <= 8192)) {
-        if (!scalarApplies(p)) return "softmaxBlockRow";
+        if (!scalarApplies(p)) {
+            if (!wideApplies(p)) return "softmaxBlockRow";
+            const WideShape f = wideShape(*p);
+            std::snprintf(name, sizeof(name), "softmaxRowWide<%s, %d, %d>", p->x_dtype == MLKD_F16 ? "_Float16" : "float",
+                          f.ch, f.w);
+            return name;
+        }
         std::snprintf(name, sizeof(name), "softmaxWaveRowScalar<%d>", ch);
         return name;
     }
@@ -417,6 +723,7 @@ extern "C" int mlkd_launch_softmax(const mlkd_softmax* p, void* stream) {
         if (p->cols <= 4096) return launchScalar<16>(*p, st);
         return launchScalar<32>(*p, st);
     }
+    if (wideApplies(p)) return launchWide(*p, st);
     int64_t blocks = p->rows < 65536 ? p->rows : 65536;
     hipLaunchKernelGGL(softmaxBlockRow, dim3(static_cast<unsigned>(blocks)), dim3(256), 0, st, *p);
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
