@@ -68,7 +68,7 @@ bool writeTextAtomic(const std::string& path, const std::string& text) {
 
 std::string num(double v) {
     char b[64];
-    std::snprintf(b, sizeof(b), "%.6g", v);
+    std::snprintf(b, sizeof(b), "%.9g", v);
     return b;
 }
 
