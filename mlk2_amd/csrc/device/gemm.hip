@@ -27,14 +27,14 @@
 // stored as loaded ([k][n]) so each MFMA operand is one conflict-free 4-byte
 // read.
 //
-// Any other shape or dtype mix runs the general tiled kernel (f32 or f64
-// accumulation, bounds-checked).
+// Any other shape or dtype mix runs the general kernels (gemm_general.hip).
 #include <hip/hip_runtime.h>
 
 #include <stdint.h>
 
 #include <algorithm>
 
+#include "gemm_general.h"
 #include "mlk_device_math.h"
 #include "runtime_abi.h"
 
@@ -1626,90 +1626,6 @@ __global__ __launch_bounds__(512, 1) void gemmF32Dma(const float* __restrict__ A
     }
 }
 
-// ------------------------------------------------------------- general ---
-template <typename T>
-__device__ __forceinline__ T ldAny(const void* p, int dt, int64_t i) {
-    if (dt == MLKD_F32) return static_cast<T>(static_cast<const float*>(p)[i]);
-    if (dt == MLKD_F16) return static_cast<T>(static_cast<float>(static_cast<const _Float16*>(p)[i]));
-    return static_cast<T>(static_cast<const double*>(p)[i]);
-}
-
-template <typename T>
-__device__ __forceinline__ void stAny(void* p, int dt, int64_t i, T v) {
-    if (dt == MLKD_F32) {
-        static_cast<float*>(p)[i] = static_cast<float>(v);
-    } else if (dt == MLKD_F16) {
-        if constexpr (sizeof(T) == sizeof(double)) static_cast<_Float16*>(p)[i] = mlk::toHalf(v);
-        else static_cast<_Float16*>(p)[i] = static_cast<_Float16>(v);
-    } else {
-        static_cast<double*>(p)[i] = static_cast<double>(v);
-    }
-}
-
-/// One 64x64 output tile by 256 threads, 4x4 per thread, K slabs of 16
-/// through LDS; k ascending per output element, starting from C's old value
-/// in the accumulate form (the reference's order, kernel_buffers.cpp:
-/// 406-432). With skip_zero_a the products of A[i,p] == 0 are left out, as
-/// there (:422).
-template <typename T>
-__device__ __forceinline__ void generalTile(const mlkd_gemm& p, int64_t row0, int64_t col0, T (&As)[16][65],
-                                            T (&Bs)[16][65]) {
-    const int tx = threadIdx.x & 15, ty = threadIdx.x >> 4;
-    T acc[4][4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t r = row0 + ty * 4 + i, c = col0 + tx * 4 + j;
-            acc[i][j] = (p.accumulate && r < p.m && c < p.n) ? ldAny<T>(p.c, p.c_dtype, r * p.ldc + c) : T(0);
-        }
-    }
-    const bool skip = p.skip_zero_a != 0;
-    for (int64_t k0 = 0; k0 < p.k; k0 += 16) {
-        for (int e = threadIdx.x; e < 16 * 64; e += 256) {
-            const int kk = e / 64, mm = e % 64;
-            const int64_t r = row0 + mm, kA = k0 + kk;
-            As[kk][mm] = (r < p.m && kA < p.k) ? ldAny<T>(p.a, p.a_dtype, r * p.lda + kA) : T(0);
-            const int64_t c = col0 + mm;
-            Bs[kk][mm] = (c < p.n && kA < p.k) ? ldAny<T>(p.b, p.b_dtype, kA * p.ldb + c) : T(0);
-        }
-        __syncthreads();
-#pragma unroll
-        for (int kk = 0; kk < 16; ++kk) {
-            T a[4], b[4];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = As[kk][ty * 4 + i];
-#pragma unroll
-            for (int j = 0; j < 4; ++j) b[j] = Bs[kk][tx * 4 + j];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                if (skip && a[i] == T(0)) continue;
-#pragma unroll
-                for (int j = 0; j < 4; ++j) acc[i][j] += a[i] * b[j];
-            }
-        }
-        __syncthreads();
-    }
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-            const int64_t r = row0 + ty * 4 + i, c = col0 + tx * 4 + j;
-            if (r < p.m && c < p.n) stAny<T>(p.c, p.c_dtype, r * p.ldc + c, acc[i][j]);
-        }
-    }
-}
-
-/// Any shape and dtype mix: one 64x64 tile per workgroup.
-template <typename T>
-__global__ __launch_bounds__(256) void gemmGeneral(mlkd_gemm p) {
-    __shared__ T As[16][65];
-    __shared__ T Bs[16][65];
-    const int64_t tilesN = (p.n + 63) / 64;
-    generalTile<T>(p, (blockIdx.x / tilesN) * 64, (blockIdx.x % tilesN) * 64, As, Bs);
-}
-
-/// Zeroes n 32-bit words.
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Process default of the f16 GEMM launch form (a launch's own `variant`
@@ -1781,6 +1697,11 @@ int mfmaForm(const mlkd_gemm* p) {
     }
     return -1;
 }
+
+/// Whether a launch runs on an MFMA form as it is. Only the accumulating
+/// (Call) form skips zeros; a non-accumulating launch that asks for the skip
+/// takes the general kernel.
+bool tiled(const mlkd_gemm* p) { return mfmaForm(p) >= 0 && (p->skip_zero_a == 0 || p->accumulate != 0); }
 
 /// Form 8 takes gemmF16Dma8s when its lane offsets fit 32 bits and
 /// gemmF16Dma8 otherwise; the two give identical results.
@@ -1888,8 +1809,7 @@ __global__ __launch_bounds__(256) void unpadBlock(const T* __restrict__ src, int
 /// The zero-padded shape a GEMM the MFMA forms do not tile runs at: f16
 /// operands with an f32 C on 256 x 256 tiles, or all-f32 on 64 x 64 tiles,
 /// K rounded up to 64. Padding adds only products 0 * 0 to the sums (and
-/// the skip-zero-A test skips them), so each output keeps its value. Below
-/// 2^30 flop the copies cost more than the general kernel takes.
+/// the skip-zero-A test skips them), so each output keeps its value.
 struct PadShape {
     int64_t m, n, k;
     size_t es;   // operand element bytes
@@ -1906,12 +1826,14 @@ bool padShape(const mlkd_gemm* p, PadShape& ps) {
     ps.n = (p->n + tn - 1) / tn * tn;
     ps.k = (p->k + tk - 1) / tk * tk;
     ps.es = f16 ? 2 : 4;
+    // A few rows or columns, padded 4 times or more in that direction alone:
+    // the general kernel fits its tiles to them (f16 64x4096x4096: 15 us
+    // against 88 us padded; 16x4096x4096: 12.5 us; f32 16x4096x4096: 17 us
+    // against 98 us).
+    if (ps.m >= 4 * p->m || ps.n >= 4 * p->n) return false;
     if (ps.m >= (int64_t{1} << 31) || ps.n >= (int64_t{1} << 31) || ps.k >= (int64_t{1} << 31)) return false;
     // Padded when the product is large (2^30 flop and up) or the padding at
-    // most 8 times the work: the general kernel takes 36 us at 100^3 and
-    // 150 us at 500^3, the padded MFMA launch tens of us at either. Thin
-    // shapes padded further (a few rows against 256-row tiles) stay on the
-    // general kernel, whose work is then small.
+    // most 8 times the work.
     const double work = static_cast<double>(p->m) * static_cast<double>(p->n) * static_cast<double>(p->k);
     const double padded = static_cast<double>(ps.m) * static_cast<double>(ps.n) * static_cast<double>(ps.k);
     return 2.0 * work >= static_cast<double>(int64_t{1} << 30) || padded <= 8.0 * work;
@@ -2037,7 +1959,9 @@ extern "C" void mlkd_gemm_set_variant(int variant) { gGemmF16Variant = variant; 
 
 extern "C" int64_t mlkd_gemm_pad_bytes(const mlkd_gemm* p) {
     PadShape ps;
-    return p != nullptr && padShape(p, ps) ? static_cast<int64_t>(padBytes(ps)) : 0;
+    if (p == nullptr) return 0;
+    if (padShape(p, ps)) return static_cast<int64_t>(padBytes(ps));
+    return tiled(p) ? 0 : mlkdGemmGeneralBytes(p);
 }
 
 extern "C" const char* mlkd_gemm_kernel_name(const mlkd_gemm* p) {
@@ -2063,8 +1987,7 @@ extern "C" const char* mlkd_gemm_kernel_name(const mlkd_gemm* p) {
         case 101: return acc ? "gemmF32Mfma<true>" : "gemmF32Mfma<false>";
         default: break;
     }
-    const bool wide = p->a_dtype == MLKD_F64 || p->b_dtype == MLKD_F64 || p->c_dtype == MLKD_F64;
-    return wide ? "gemmGeneral<double>" : "gemmGeneral<float>";
+    return mlkdGemmGeneralName(p);
 }
 
 extern "C" int mlkd_launch_gemm(const mlkd_gemm* p, void* stream) {
@@ -2074,11 +1997,7 @@ extern "C" int mlkd_launch_gemm(const mlkd_gemm* p, void* stream) {
     // The MFMA forms take the skip-zero-A Call form themselves: a wave whose
     // accumulators met an infinity or a NaN recomputes its block exactly. One
     // launch, no scratch, no host read-back.
-    // Only the accumulating (Call) form skips; a non-accumulating launch that
-    // asks for the skip takes the general kernel.
-    if (const int form = mfmaForm(p); form >= 0 && (p->skip_zero_a == 0 || p->accumulate != 0)) {
-        return launchMfma(p, form, st);
-    }
+    if (tiled(p)) return launchMfma(p, mfmaForm(p), st);
     {
         mlkd_gemm q;
         PadShape ps;
@@ -2087,13 +2006,5 @@ extern "C" int mlkd_launch_gemm(const mlkd_gemm* p, void* stream) {
             return launchPadded(p, q, ps, st);
         }
     }
-    const int64_t tiles = ((p->m + 63) / 64) * ((p->n + 63) / 64);
-    if (tiles > 0x7FFFFFFF) return MLKD_RT_LAUNCH;
-    const bool wide = p->a_dtype == MLKD_F64 || p->b_dtype == MLKD_F64 || p->c_dtype == MLKD_F64;
-    if (wide) {
-        hipLaunchKernelGGL(gemmGeneral<double>, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, st, *p);
-    } else {
-        hipLaunchKernelGGL(gemmGeneral<float>, dim3(static_cast<unsigned>(tiles)), dim3(256), 0, st, *p);
-    }
-    return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
+    return mlkdLaunchGemmGeneral(p, st);
 }

@@ -52,8 +52,9 @@ typedef struct mlkd_gemm {
     int32_t pad_;
     /* Device workspace for shapes the MFMA forms do not tile
        (mlkd_gemm_pad_bytes): the operands are copied into zero-padded
-       blocks there, the MFMA form runs on them and C is copied back. NULL
-       (or too small) keeps such shapes on the general kernel. */
+       blocks there, the MFMA form runs on them and C is copied back; or the
+       general kernel's K ranges leave their sums there. NULL (or too small)
+       runs such shapes on the general kernel in one range. */
     void* work;
     int64_t work_bytes;
 } mlkd_gemm;

@@ -362,8 +362,9 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
         case StepKind::Gemm: {
             // f16 x f16 -> f32 with M, N % 256 and K % 64 runs the MFMA forms
             // on 256 x 256 tiles (forms 5 and 6: 128 x 256); f32 with M, N % 64
-            // and K % 32 the 64 x 64 MFMA tiles; anything else the
-            // bounds-checked 64 x 64 general kernel.
+            // and K % 32 the 64 x 64 MFMA tiles (on padded copies where
+            // that pays); anything else the bounds-checked general kernel,
+            // on tiles it fits to the shape.
             instances = st.m * st.n;
             auto dt = [&](uint32_t b) { return km.buffers[b].dtype; };
             const bool f16 = dt(st.a) == Dtype::F16 && dt(st.b) == Dtype::F16 && dt(st.c) == Dtype::F32 &&
@@ -376,7 +377,28 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
             perGroup = tm * tn;
             covered = workgroups * perGroup >= instances;
             form = f16 ? (half ? "128 x 256 output tiles, two workgroups per CU" : "256 x 256 output tiles")
-                       : f32 ? "64 x 64 output tiles" : "64 x 64 output tiles, bounds-checked";
+                       : "64 x 64 output tiles";
+            if (!f16 && !f32) {
+                auto code = [](Dtype d) { return d == Dtype::F32 ? MLKD_F32 : d == Dtype::F16 ? MLKD_F16 : MLKD_F64; };
+                mlkd_gemm p{};
+                p.a_dtype = code(dt(st.a));
+                p.b_dtype = code(dt(st.b));
+                p.c_dtype = code(dt(st.c));
+                p.accumulate = st.accumulate ? 1 : 0;
+                p.skip_zero_a = st.skipZeroA && st.k > 0 ? 1 : 0;
+                p.m = st.m;
+                p.n = st.n;
+                p.k = st.k;
+                p.lda = st.lda;
+                p.ldb = st.ldb;
+                p.ldc = st.ldc;
+                p.variant = -1;
+                int64_t rows = 0, cols = 0;
+                mlkd_gemm_general_tile(&p, &rows, &cols, &workgroups);
+                perGroup = rows * cols;
+                covered = workgroups * perGroup >= instances;
+                form = "output tiles fitted to the shape, bounds-checked";
+            }
             break;
         }
         case StepKind::ScoreSoftmax: {
