@@ -33,6 +33,7 @@
 #include <stdint.h>
 
 #include <algorithm>
+#include <type_traits>
 
 #include "gemm_general.h"
 #include "mlk_device_math.h"
@@ -1197,6 +1198,66 @@ __device__ __forceinline__ void dmaLoad16s(const void* sbase, uint32_t voff, uin
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(voff), "s"(sbase), "s"(m0) : "memory");
 }
 
+// ---------------------------------------------------------- f16 ragged ----
+/// Operands of a ragged member (form 8, f32 form 0): C is m x n; A's rows hold
+/// ka columns (k, or k rounded up with zeros), B's nb columns (n, or n rounded
+/// up), both whole 16-byte pieces at 16-byte aligned rows.
+template <typename T>
+struct Ragged {
+    const T* a;
+    const T* b;
+    float* c;
+    int m, n, k, ka, nb;
+    int tilesM, tilesN;
+    int64_t lda, ldb, ldc;
+    int skip;
+};
+using RaggedF16 = Ragged<_Float16>;
+using RaggedF32 = Ragged<float>;
+
+__device__ __align__(16) const uint32_t kZero16[4] = {0u, 0u, 0u, 0u};
+
+/// exactWaveBlock bounded to m x n.
+template <typename T>
+__device__ __forceinline__ void exactRaggedBlock(const Ragged<T>& p, int r0, int c0, int rows, int cols) {
+    const int lane = threadIdx.x & 63;
+    rows = min(rows, p.m - r0);
+    cols = min(cols, p.n - c0);
+    if (lane >= cols) return;
+    for (int r = 0; r < rows; ++r) {
+        const T* a = p.a + (r0 + r) * p.lda;
+        float* dst = p.c + (r0 + r) * p.ldc + c0 + lane;
+        float s = *dst;
+        for (int k = 0; k < p.k; ++k) {
+            const float av = static_cast<float>(a[k]);
+            if (av != 0.0f) s = s + av * static_cast<float>(p.b[k * p.ldb + c0 + lane]);
+        }
+        *dst = s;
+    }
+}
+
+/// 16 bytes at 4-byte alignment, all a ragged C has.
+struct __attribute__((packed, aligned(4))) Row4 {
+    f32x4 v;
+};
+
+__device__ __forceinline__ f32x4 loadAny16(const float* p) { return reinterpret_cast<const Row4*>(p)->v; }
+
+/// v (+)= into columns col..col+3 of a row of n.
+template <bool ACC>
+__device__ __forceinline__ void storeRagged(float* row, int col, int n, f32x4 v) {
+    float* dst = row + col;
+    if (col + 4 <= n) {
+        if (ACC) v += reinterpret_cast<const Row4*>(dst)->v;
+        reinterpret_cast<Row4*>(dst)->v = v;
+    } else {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            if (col + e < n) dst[e] = ACC ? dst[e] + v[e] : v[e];
+        }
+    }
+}
+
 /// Variant 8 (K a multiple of 64): the same tiles, ring, swizzles and
 /// per-accumulator MFMAs as gemmF16Dma8 (results identical bit for bit), with
 /// no per-step vector address arithmetic and a fixed instruction order.
@@ -1224,35 +1285,47 @@ __device__ __forceinline__ void dmaLoad16s(const void* sbase, uint32_t voff, uin
 ///   consecutive MFMAs share an operand register (0.8% faster than plain
 ///   row order, identical results).
 /// Needs lda < 2^23 and ldb < 2^25 (32-bit lane offsets).
-template <bool ACC>
-__global__ __launch_bounds__(512, 1) void gemmF16Dma8s(const _Float16* __restrict__ A,
-                                                       const _Float16* __restrict__ B,
-                                                       float* __restrict__ C, int M, int N, int K,
-                                                       int64_t lda, int64_t ldb, int64_t ldc,
-                                                       int skipZeroA) {
+/// RAGGED: any m and n, k of any length (rag holds the rest of it); rows past
+/// m and columns past n repeat the last ones and are not stored, and lanes
+/// past k load zeros in the last K step.
+template <bool ACC, bool RAGGED>
+__device__ __forceinline__ void dma8sTile(const _Float16* __restrict__ A, const _Float16* __restrict__ B,
+                                          float* __restrict__ C, int M, int N, int K, int64_t lda, int64_t ldb,
+                                          int64_t ldc, int skipZeroA, const RaggedF16& rag) {
     extern __shared__ __align__(16) _Float16 lds[];
     const int lane = threadIdx.x & 63;
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int wm = wave >> 2, wn = wave & 3;
     int tm, tn;
-    xcdTile(M / kBM, N / kBN, tm, tn);
+    if constexpr (RAGGED) xcdTile(rag.tilesM, rag.tilesN, tm, tn);
+    else xcdTile(M / kBM, N / kBN, tm, tn);
     const int64_t row0 = static_cast<int64_t>(tm) * kBM;
     const int64_t col0 = static_cast<int64_t>(tn) * kBN;
-    const int steps = K / kDmaBK;
+    const int steps = RAGGED ? (K + kDmaBK - 1) / kDmaBK : K / kDmaBK;
+    const bool partial = RAGGED && K % kDmaBK != 0;
 
     // Wave w's direct loads are A instructions 2w, 2w + 1 (16 rows each) and
     // B instructions 2w, 2w + 1 (2 k-rows each) of every stage, as in
     // gemmF16Dma8: lane byte offsets from the tile's A rows / B columns.
     uint32_t gA[2], gB[2];
+    int kA[2], kB[2];   // RAGGED: first k of the lane's A piece, k of its B piece, in a step
 #pragma unroll
     for (int j = 0; j < 2; ++j) {
         const int q = (wave * 2 + j) * 64 + lane;
         const int row = q >> 2;
         const int c = (q & 3) ^ ((row >> 2) & 3);
-        gA[j] = static_cast<uint32_t>((row * lda + c * 8) * 2);
         const int krow = q >> 5;
         const int cb = (q & 31) ^ ((krow & 3) * 4);
-        gB[j] = static_cast<uint32_t>((krow * ldb + cb * 8) * 2);
+        if constexpr (RAGGED) {
+            const int r0 = static_cast<int>(row0), c0 = static_cast<int>(col0);
+            gA[j] = static_cast<uint32_t>(((min(r0 + row, M - 1) - r0) * lda + c * 8) * 2);
+            gB[j] = static_cast<uint32_t>((krow * ldb + min(c0 + cb * 8, rag.nb - 8) - c0) * 2);
+        } else {
+            gA[j] = static_cast<uint32_t>((row * lda + c * 8) * 2);
+            gB[j] = static_cast<uint32_t>((krow * ldb + cb * 8) * 2);
+        }
+        kA[j] = c * 8;
+        kB[j] = krow;
     }
     const char* aTile = reinterpret_cast<const char*>(A + row0 * lda);
     const char* bTile = reinterpret_cast<const char*>(B + col0);
@@ -1261,6 +1334,20 @@ __global__ __launch_bounds__(512, 1) void gemmF16Dma8s(const _Float16* __restric
     // Direct load j (A 0, A 1, B 0, B 1) of stage t (K step min(t, steps - 1))
     // into ring slot `slot` = t % 4.
     auto issueOne = [&](int t, const int slot, const int j) {
+        if constexpr (RAGGED) {
+            if (partial && t >= steps - 1) {
+                const int s = steps - 1;
+                const char* src = j < 2 ? aTile + static_cast<int64_t>(s) * (kDmaBK * 2) + gA[j & 1]
+                                        : bTile + s * ldb * (kDmaBK * 2) + gB[j & 1];
+                if ((j < 2 ? kA[j & 1] : kB[j & 1]) >= (j < 2 ? rag.ka : K) - s * kDmaBK) {
+                    src = reinterpret_cast<const char*>(kZero16);
+                }
+                const uint32_t m = m0Wave + static_cast<uint32_t>(slot) * (kDmaStage * 2u) + (j & 1) * 1024u +
+                                   (j >= 2 ? kDmaA * 2u : 0u);
+                asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m) : "memory");
+                return;
+            }
+        }
         const int64_t k0 = static_cast<int64_t>(min(t, steps - 1)) * kDmaBK;
         const char* a = aTile + k0 * 2;
         const char* b = bTile + k0 * ldb * 2;
@@ -1369,12 +1456,32 @@ __global__ __launch_bounds__(512, 1) void gemmF16Dma8s(const _Float16* __restric
         step(s + 2, 2, bX, bY);
         step(s + 3, 3, bY, bX);
     }
-    if (s < steps) {   // K % 128 == 64: two more steps, in slots 0 and 1
+    if constexpr (RAGGED) {
+        if (s < steps) step(s, 0, bX, bY);
+        if (s + 1 < steps) step(s + 1, 1, bY, bX);
+        if (s + 2 < steps) step(s + 2, 2, bX, bY);
+    } else if (s < steps) {   // K % 128 == 64: two more steps, in slots 0 and 1
         step(s, 0, bX, bY);
         step(s + 1, 1, bY, bX);
     }
     // No direct load may still be writing LDS when the workgroup ends.
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    if constexpr (RAGGED) {
+        const int r0 = static_cast<int>(row0) + wm * 128, c0 = static_cast<int>(col0) + wn * 64;
+        if (ACC && skipZeroA && waveNonFinite(acc)) {
+            exactRaggedBlock(rag, r0, c0, 128, 64);
+            return;
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const int row = r0 + i * 16 + l16;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                if (row < M) storeRagged<ACC>(C + row * ldc, c0 + j * 16 + 4 * g, N, acc[i][j]);
+            }
+        }
+        return;
+    }
     if (ACC && skipZeroA && waveNonFinite(acc)) {
         exactWaveBlock<_Float16, _Float16>(A, B, C, lda, ldb, ldc, K, row0 + wm * 128, col0 + wn * 64, 128, 64, ACC);
         return;
@@ -1388,6 +1495,201 @@ __global__ __launch_bounds__(512, 1) void gemmF16Dma8s(const _Float16* __restric
             f32x4 v = acc[i][j];
             if (ACC) v += *dst;
             *dst = v;
+        }
+    }
+}
+
+template <bool ACC>
+__global__ __launch_bounds__(512, 1) void gemmF16Dma8s(const _Float16* __restrict__ A,
+                                                       const _Float16* __restrict__ B,
+                                                       float* __restrict__ C, int M, int N, int K,
+                                                       int64_t lda, int64_t ldb, int64_t ldc,
+                                                       int skipZeroA) {
+    dma8sTile<ACC, false>(A, B, C, M, N, K, lda, ldb, ldc, skipZeroA, RaggedF16{});
+}
+
+/// The ragged member on the same 256 x 256 tiles.
+struct RaggedF16Wide : RaggedF16 {};
+
+template <bool ACC>
+__global__ __launch_bounds__(512, 1) void gemmF16Dma8s(RaggedF16Wide p) {
+    dma8sTile<ACC, true>(p.a, p.b, p.c, p.m, p.n, p.k, p.lda, p.ldb, p.ldc, p.skip, p);
+}
+
+constexpr int kRM = 128, kRN = 128;                        // output tile
+constexpr int kRA = kRM * kDmaBK;                          // halves per A stage
+constexpr int kRStage = kRA + kDmaBK * kRN;                // A, then B
+constexpr size_t kLdsRagged = static_cast<size_t>(kDmaStages) * kRStage * sizeof(_Float16);   // 64 KiB
+
+/// The ragged member on tiles of 128 x 128, for shapes that 256 x 256 tiles
+/// leave most of the chip idle with: the same direct loads, ring, swizzles,
+/// MFMAs and fences, 4 waves of 64 x 64 (16 MFMAs a K step), two workgroups to
+/// a CU, bounded as dma8sTile<ACC, true> is. A K step takes 0.31 us for each
+/// tile on a CU, one or two: its LDS traffic (32 KiB of reads, half of them
+/// transposed, 16 KiB of direct loads; 256 x 128 tiles of 8 waves, a quarter
+/// less to load, are no faster). 2000 x 1000 x 3000 takes 24.5 us, with C += A
+/// B 27.9 us (zero-padded copies of A, B and C around 256 x 256 tiles: 44.4
+/// and 59.7 us), 2000^3 25 us (58 us), 1000 x 600 x 1000 10.4 us (28 us).
+template <bool ACC>
+__global__ __launch_bounds__(256, 2) void gemmF16Dma8s(RaggedF16 p) {
+    extern __shared__ __align__(16) _Float16 lds[];
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
+    const int wm = wave >> 1, wn = wave & 1;
+    // Consecutive workgroups go to different XCDs: each takes a contiguous
+    // share of the tiles, in columns of 8 tile rows, so that its L2 holds 8 A
+    // panels and few B panels.
+    const int total = p.tilesM * p.tilesN;
+    int id = static_cast<int>(blockIdx.x);
+    if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
+    const int band = id / (8 * p.tilesN), inBand = id % (8 * p.tilesN);
+    const int bandRows = min(8, p.tilesM - band * 8);
+    const int tm = band * 8 + inBand % bandRows, tn = inBand / bandRows;
+    const int row0 = tm * kRM, col0 = tn * kRN;
+    const int steps = (p.k + kDmaBK - 1) / kDmaBK;
+    const bool partial = p.k % kDmaBK != 0;
+
+    // Wave w's direct loads are A instructions 2w, 2w + 1 (16 rows each) and
+    // B instructions 2w, 2w + 1 (4 k-rows each) of every stage.
+    uint32_t gA[2], gB[2];
+    int kA[2], kB[2];   // first k of the lane's A piece, k of its B piece, in a step
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const int q = (wave * 2 + j) * 64 + lane;
+        const int row = q >> 2;
+        kA[j] = ((q & 3) ^ ((row >> 2) & 3)) * 8;
+        gA[j] = static_cast<uint32_t>(((min(row0 + row, p.m - 1) - row0) * p.lda + kA[j]) * 2);
+        kB[j] = q >> 4;
+        const int col = ((q & 15) ^ ((kB[j] & 3) * 4)) * 8;
+        gB[j] = static_cast<uint32_t>((kB[j] * p.ldb + min(col0 + col, p.nb - 8) - col0) * 2);
+    }
+    const char* aTile = reinterpret_cast<const char*>(p.a + row0 * p.lda);
+    const char* bTile = reinterpret_cast<const char*>(p.b + col0);
+    const uint32_t ldsS = __builtin_amdgcn_readfirstlane(ldsOffset(lds));
+    const uint32_t m0Wave = ldsS + static_cast<uint32_t>(wave) * 2048u;
+    // Direct load j (A 0, A 1, B 0, B 1) of stage t (K step min(t, steps - 1))
+    // into ring slot `slot`.
+    auto issueOne = [&](int t, const int slot, const int j) {
+        const int s = min(t, steps - 1);
+        const char* a = aTile + static_cast<int64_t>(s) * (kDmaBK * 2);
+        const char* b = bTile + s * p.ldb * (kDmaBK * 2);
+        const uint32_t m = m0Wave + static_cast<uint32_t>(slot) * (kRStage * 2u) + (j & 1) * 1024u +
+                           (j >= 2 ? kRA * 2u : 0u);
+        if (partial && s == steps - 1) {
+            const int left = (j < 2 ? p.ka : p.k) - s * kDmaBK;
+            const char* src = j < 2 ? a + gA[j & 1] : b + gB[j & 1];
+            if ((j < 2 ? kA[j & 1] : kB[j & 1]) >= left) src = reinterpret_cast<const char*>(kZero16);
+            asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" ::"v"(src), "s"(m) : "memory");
+        } else {
+            dmaLoad16s(j < 2 ? a : b, j < 2 ? gA[j & 1] : gB[j & 1], m);
+        }
+    };
+    f32x4 acc[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) acc[i][j] = f32x4{0.0f, 0.0f, 0.0f, 0.0f};
+    }
+#pragma unroll
+    for (int t = 0; t < 3; ++t) {
+#pragma unroll
+        for (int j = 0; j < 4; ++j) issueOne(t, t, j);
+    }
+    // Fragment bases; the slot (16 KiB), the m-tile (1 KiB) and the second
+    // transposed half (4 k-rows, 1 KiB) are immediates.
+    const int l16 = lane & 15, g = lane >> 4;
+    uint32_t vA;
+    {
+        const int row = wm * 64 + l16;
+        vA = ldsS + 2u * (row * kDmaBK + ((g ^ ((row >> 2) & 3)) * 8));
+    }
+    uint32_t vB[4];
+#pragma unroll
+    for (int nt = 0; nt < 4; ++nt) {
+        const int krow = 8 * g + (l16 >> 2);
+        const int col = wn * 64 + nt * 16 + 4 * (l16 & 3);
+        vB[nt] = ldsS + 2u * (kRA + krow * kRN + (((col >> 3) ^ ((krow & 3) * 4)) * 8) + (col & 7));
+    }
+    auto readA = [&](f16x8& f, const int slot, int mt) {
+        f = *reinterpret_cast<const __attribute__((address_space(3))) f16x8*>(
+            vA + static_cast<uint32_t>(slot * kRStage * 2 + 1024 * mt));
+    };
+    auto readB = [&](f16x8& f, const int slot, int nt) {
+        const uint32_t base = vB[nt] + static_cast<uint32_t>(slot * kRStage * 2);
+        const fp16x4 v0 = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+            reinterpret_cast<__attribute__((address_space(3))) fp16x4*>(base));
+        const fp16x4 v1 = __builtin_amdgcn_ds_read_tr16_b64_v4f16(
+            reinterpret_cast<__attribute__((address_space(3))) fp16x4*>(base + 1024u));
+        f = __builtin_shufflevector(__builtin_bit_cast(f16x4, v0), __builtin_bit_cast(f16x4, v1), 0, 1, 2, 3, 4, 5,
+                                    6, 7);
+    };
+    f16x8 aX[4], aY[4], bX[4], bY[4];
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+#pragma unroll
+    for (int i = 0; i < 4; ++i) readA(aX[i], 0, i);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) readB(bX[j], 0, j);
+    // K step s in ring slot q = s % 4: 6 MFMAs, then the barrier that
+    // certifies stage s + 1 (one later stage may be in flight) and frees slot
+    // (s - 1) % 4, then step s + 1's fragments and stage s + 3's loads behind
+    // the other MFMAs.
+    auto step = [&](int s, const int q, f16x8 (&a)[4], f16x8 (&b)[4], f16x8 (&an)[4], f16x8 (&bn)[4]) {
+        const int qn = (q + 1) & 3;
+#pragma unroll
+        for (int idx = 0; idx < 16; ++idx) {
+            const int mi = idx >> 2, ni = (mi & 1) ? 3 - (idx & 3) : (idx & 3);
+            acc[mi][ni] = __builtin_amdgcn_mfma_f32_16x16x32_f16(b[ni], a[mi], acc[mi][ni], 0, 0, 0);
+            if (idx == 5) {
+                asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+                asm volatile("s_barrier" ::: "memory");
+            }
+            if (idx == 6) readB(bn[0], qn, 0);
+            if (idx == 7) readA(an[0], qn, 0);
+            if (idx >= 8 && idx <= 10) readB(bn[idx - 7], qn, idx - 7);
+            if (idx >= 11 && idx <= 13) readA(an[idx - 10], qn, idx - 10);
+            if (idx >= 12) issueOne(s + 3, (q + 3) & 3, idx - 12);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    };
+    int s = 0;
+    for (; s + 4 <= steps; s += 4) {
+        step(s, 0, aX, bX, aY, bY);
+        step(s + 1, 1, aY, bY, aX, bX);
+        step(s + 2, 2, aX, bX, aY, bY);
+        step(s + 3, 3, aY, bY, aX, bX);
+    }
+    if (s < steps) step(s, 0, aX, bX, aY, bY);
+    if (s + 1 < steps) step(s + 1, 1, aY, bY, aX, bX);
+    if (s + 2 < steps) step(s + 2, 2, aX, bX, aY, bY);
+    // No direct load may still be writing LDS when the workgroup ends.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    const int r0 = row0 + wm * 64, c0 = col0 + wn * 64;
+    if (ACC && p.skip && waveNonFinite(acc)) {
+        exactRaggedBlock(p, r0, c0, 64, 64);
+        return;
+    }
+    // C += reads all of the wave's C before its first store: the reads of a
+    // few, each waited for, took 6 us more at 1000 x 600 x 1000.
+    f32x4 old[4][4];
+    if constexpr (ACC) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const float* row = p.c + min(r0 + i * 16 + l16, p.m - 1) * p.ldc;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) old[i][j] = loadAny16(row + min(c0 + j * 16 + 4 * g, p.n - 4));
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int row = r0 + i * 16 + l16;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const int col = c0 + j * 16 + 4 * g;
+            if (row >= p.m) continue;
+            float* dst = p.c + row * p.ldc;
+            if (ACC && col + 4 <= p.n) storeRagged<false>(dst, col, p.n, acc[i][j] + old[i][j]);
+            else storeRagged<ACC>(dst, col, p.n, acc[i][j]);
         }
     }
 }
@@ -1626,6 +1928,105 @@ __global__ __launch_bounds__(512, 1) void gemmF32Dma(const float* __restrict__ A
     }
 }
 
+/// The ragged member: the same ring and reads on any m, n and k. Rows past m
+/// and columns past n repeat the last ones and are not stored; in the last K
+/// step, lanes past k load zeros. (A text of its own: a shared one moves the
+/// instructions of the whole-block kernel, 1% at 1024^3.) 1000^3 takes 22.9
+/// us, 700 x 1000 x 900 with C += A B 24.4 us (zero-padded copies of A, B and C
+/// around the whole-block kernel: 30.0 and 36.0 us).
+template <bool ACC>
+__global__ __launch_bounds__(512, 1) void gemmF32Dma(RaggedF32 p) {
+    extern __shared__ __align__(16) float ldsF[];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int quad = wave & 3, h = wave >> 2;   // output quadrant, K-step half
+    const int wm = quad >> 1, wn = quad & 1;
+    int tm, tn;
+    xcdTile(p.tilesM, p.tilesN, tm, tn);
+    const int row0 = tm * kFM, col0 = tn * kFN;
+    const int steps = (p.k + kQK - 1) / kQK;
+    auto issue = [&](int slot) {
+        const int k0 = min(slot, steps - 1) * kQK;
+        const float* st = ldsF + (slot % kQStages) * kQStage;
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int ins = wave * 2 + j;
+            const int row = ins * 4 + (lane >> 4);
+            const int k = k0 + ((lane & 15) ^ (row & 15)) * 4;
+            const void* src = p.a + min(row0 + row, p.m - 1) * p.lda + k;
+            if (k >= p.ka) src = kZero16;
+            dmaLoad16(static_cast<const _Float16*>(src), reinterpret_cast<const _Float16*>(st + ins * 256));
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int ins = wave * 2 + j;
+            const int k = k0 + ins * 4 + (lane >> 4);
+            const void* src = p.b + k * p.ldb + min(col0 + (lane & 15) * 4, p.nb - 4);
+            if (k >= p.k) src = kZero16;
+            dmaLoad16(static_cast<const _Float16*>(src), reinterpret_cast<const _Float16*>(st + kQA + ins * 256));
+        }
+    };
+    f32x16 acc;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] = 0.0f;
+#pragma unroll
+    for (int s = 0; s < kQStages - 1; ++s) issue(s);
+    const int l32 = lane & 31, hl = lane >> 5;
+    const int m = wm * 32 + l32;
+    uint32_t offA[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int q = 4 * h + i;
+        offA[i] = 4u * static_cast<uint32_t>(m * kQK + (((8 * hl + q) ^ (m & 15)) * 4));
+    }
+    const uint32_t offB = 4u * static_cast<uint32_t>(kQA + (32 * hl + 16 * h) * kFN + wn * 32 + l32);
+    const uint32_t ldsBase = ldsOffset(ldsF);
+    asm volatile("s_waitcnt vmcnt(8)" ::: "memory");
+    asm volatile("s_barrier" ::: "memory");
+    for (int s = 0; s < steps; ++s) {
+        const uint32_t cb = ldsBase + 4u * static_cast<uint32_t>((s % kQStages) * kQStage);
+        f32x4 a[4];
+        float b[16];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) a[i] = *reinterpret_cast<const __attribute__((address_space(3))) f32x4*>(cb + offA[i]);
+#pragma unroll
+        for (int t = 0; t < 16; ++t) {
+            b[t] = *reinterpret_cast<const __attribute__((address_space(3))) float*>(cb + offB + 4u * kFN * t);
+        }
+#pragma unroll
+        for (int t = 0; t < 16; ++t) acc = __builtin_amdgcn_mfma_f32_32x32x2f32(a[t >> 2][t & 3], b[t], acc, 0, 0, 0);
+        asm volatile("s_waitcnt vmcnt(4)" ::: "memory");
+        asm volatile("s_barrier" ::: "memory");
+        issue(s + kQStages - 1);
+    }
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    float* red = ldsF + quad * (64 * 16);
+    if (h == 1) {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) red[r * 64 + lane] = acc[r];
+    }
+    __syncthreads();
+    if (h == 1) return;
+#pragma unroll
+    for (int r = 0; r < 16; ++r) acc[r] += red[r * 64 + lane];
+    const int r0 = row0 + wm * 32, c0 = col0 + wn * 32;
+    if (ACC && p.skip && waveNonFinite(acc)) {
+        exactRaggedBlock(p, r0, c0, 32, 32);
+        return;
+    }
+    const int col = c0 + l32;
+    auto rowOf = [&](int r) { return r0 + 8 * (r >> 2) + 4 * hl + (r & 3); };
+    if (ACC) {   // all of the lane's C before its first store
+        const float* old = p.c + min(col, p.n - 1);
+#pragma unroll
+        for (int r = 0; r < 16; ++r) acc[r] += old[min(rowOf(r), p.m - 1) * p.ldc];
+    }
+#pragma unroll
+    for (int r = 0; r < 16; ++r) {
+        if (rowOf(r) < p.m && col < p.n) p.c[rowOf(r) * p.ldc + col] = acc[r];
+    }
+}
+
 bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) == 0; }
 
 // Process default of the f16 GEMM launch form (a launch's own `variant`
@@ -1636,6 +2037,14 @@ bool aligned16(const void* p) { return (reinterpret_cast<uintptr_t>(p) & 15u) ==
 // 8: variant 7's data path with 8 waves of 16x16x32 MFMA tiles (measured
 // fastest on gfx950).
 int gGemmF16Variant = 8;
+
+/// The members of gemmF16Dma8s: whole 256 x 256 x 64 blocks, and ragged shapes.
+using Tiled8s = void (*)(const _Float16*, const _Float16*, float*, int, int, int, int64_t, int64_t, int64_t, int);
+using Ragged8s = void (*)(RaggedF16);
+using RaggedWide8s = void (*)(RaggedF16Wide);
+/// And of gemmF32Dma.
+using TiledF32 = void (*)(const float*, const float*, float*, int, int, int64_t, int64_t, int64_t, int);
+using RaggedDma = void (*)(RaggedF32);
 
 /// Raises the dynamic-LDS limit of every form that needs more than the
 /// default, once per process (a function-local static: its initialization
@@ -1661,10 +2070,14 @@ int raiseLdsLimits() {
             {reinterpret_cast<const void*>(gemmF16Dma<false>), kLdsDma},
             {reinterpret_cast<const void*>(gemmF16Dma8<true>), kLdsDma},
             {reinterpret_cast<const void*>(gemmF16Dma8<false>), kLdsDma},
-            {reinterpret_cast<const void*>(gemmF16Dma8s<true>), kLdsDma},
-            {reinterpret_cast<const void*>(gemmF16Dma8s<false>), kLdsDma},
-            {reinterpret_cast<const void*>(gemmF32Dma<true>), kLdsF32Dma},
-            {reinterpret_cast<const void*>(gemmF32Dma<false>), kLdsF32Dma},
+            {reinterpret_cast<const void*>(static_cast<Tiled8s>(gemmF16Dma8s<true>)), kLdsDma},
+            {reinterpret_cast<const void*>(static_cast<Tiled8s>(gemmF16Dma8s<false>)), kLdsDma},
+            {reinterpret_cast<const void*>(static_cast<RaggedWide8s>(gemmF16Dma8s<true>)), kLdsDma},
+            {reinterpret_cast<const void*>(static_cast<RaggedWide8s>(gemmF16Dma8s<false>)), kLdsDma},
+            {reinterpret_cast<const void*>(static_cast<TiledF32>(gemmF32Dma<true>)), kLdsF32Dma},
+            {reinterpret_cast<const void*>(static_cast<TiledF32>(gemmF32Dma<false>)), kLdsF32Dma},
+            {reinterpret_cast<const void*>(static_cast<RaggedDma>(gemmF32Dma<true>)), kLdsF32Dma},
+            {reinterpret_cast<const void*>(static_cast<RaggedDma>(gemmF32Dma<false>)), kLdsF32Dma},
         };
         for (const Need& n : needs) {
             if (hipFuncSetAttribute(n.fn, hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(n.bytes)) !=
@@ -1723,8 +2136,9 @@ int launchMfma(const mlkd_gemm* p, int form, hipStream_t st) {
     switch (form) {
         case 8:
             if (scalarAddressed8(p)) {
-                hipLaunchKernelGGL((acc ? gemmF16Dma8s<true> : gemmF16Dma8s<false>), dim3(tiles), dim3(512), kLdsDma,
-                                   st, a16, b16, c, m, n, k, p->lda, p->ldb, p->ldc, skip);
+                const Tiled8s kern = acc ? Tiled8s{gemmF16Dma8s<true>} : Tiled8s{gemmF16Dma8s<false>};
+                hipLaunchKernelGGL(kern, dim3(tiles), dim3(512), kLdsDma, st, a16, b16, c, m, n, k, p->lda, p->ldb,
+                                   p->ldc, skip);
             } else {
                 hipLaunchKernelGGL((acc ? gemmF16Dma8<true> : gemmF16Dma8<false>), dim3(tiles), dim3(512), kLdsDma,
                                    st, a16, b16, c, m, n, k, p->lda, p->ldb, p->ldc, skip);
@@ -1766,8 +2180,8 @@ int launchMfma(const mlkd_gemm* p, int form, hipStream_t st) {
             const float* a32 = static_cast<const float*>(p->a);
             const float* b32 = static_cast<const float*>(p->b);
             if (form == 100) {
-                hipLaunchKernelGGL((acc ? gemmF32Dma<true> : gemmF32Dma<false>), dim3(ftiles), dim3(512), kLdsF32Dma,
-                                   st, a32, b32, c, n, k, p->lda, p->ldb, p->ldc, skip);
+                hipLaunchKernelGGL((acc ? TiledF32{gemmF32Dma<true>} : TiledF32{gemmF32Dma<false>}), dim3(ftiles), dim3(512),
+                                   kLdsF32Dma, st, a32, b32, c, n, k, p->lda, p->ldb, p->ldc, skip);
             } else {
                 hipLaunchKernelGGL((acc ? gemmF32Mfma<true> : gemmF32Mfma<false>), dim3(ftiles), dim3(256), 0, st,
                                    a32, b32, c, m, n, k, p->lda, p->ldb, p->ldc, p->accumulate, skip);
@@ -1780,175 +2194,158 @@ int launchMfma(const mlkd_gemm* p, int form, hipStream_t st) {
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
 }
 
-/// dst[r, c] = src[r * lds + c] for r < rows, c < cols, and 0 on the rest
-/// of the drows x dcols block (row-major, stride dcols). Element bits are
-/// copied as they are (T is a 16- or 32-bit integer type).
-template <typename T>
-__global__ __launch_bounds__(256) void padBlock(const T* __restrict__ src, int64_t rows, int64_t cols,
-                                                int64_t lds, T* __restrict__ dst, int64_t drows, int64_t dcols) {
-    for (int64_t r = blockIdx.y; r < drows; r += gridDim.y) {
-        for (int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; c < dcols;
-             c += static_cast<int64_t>(gridDim.x) * 256) {
-            dst[r * dcols + c] = (r < rows && c < cols) ? src[r * lds + c] : T(0);
-        }
-    }
-}
-
-/// dst[r * ldd + c] = src[r * scols + c] for r < rows, c < cols.
-template <typename T>
-__global__ __launch_bounds__(256) void unpadBlock(const T* __restrict__ src, int64_t scols, T* __restrict__ dst,
-                                                  int64_t rows, int64_t cols, int64_t ldd) {
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-        for (int64_t c = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; c < cols;
-             c += static_cast<int64_t>(gridDim.x) * 256) {
-            dst[r * ldd + c] = src[r * scols + c];
-        }
-    }
-}
-
-/// The zero-padded shape a GEMM the MFMA forms do not tile runs at: f16
-/// operands with an f32 C on 256 x 256 tiles, or all-f32 on 64 x 64 tiles,
-/// K rounded up to 64. Padding adds only products 0 * 0 to the sums (and
-/// the skip-zero-A test skips them), so each output keeps its value.
-struct PadShape {
-    int64_t m, n, k;
-    size_t es;   // operand element bytes
-};
-
-bool padShape(const mlkd_gemm* p, PadShape& ps) {
+/// Whether a product no whole-block form tiles runs on a ragged member: f16
+/// operands with an f32 C, or all-f32, at least 2^30 flop or a padding to 256 x
+/// 256 (f32: 64 x 64) x 64 blocks of at most 8 times the work. The general
+/// kernel has the others.
+bool raggedShape(const mlkd_gemm* p) {
     const bool f16 = p->a_dtype == MLKD_F16 && p->b_dtype == MLKD_F16 && p->c_dtype == MLKD_F32;
     const bool f32 = p->a_dtype == MLKD_F32 && p->b_dtype == MLKD_F32 && p->c_dtype == MLKD_F32;
     if (!(f16 || f32) || p->m <= 0 || p->n <= 0 || p->k <= 0) return false;
     if (p->skip_zero_a != 0 && p->accumulate == 0) return false;   // that launch takes the general kernel
-    if (mfmaForm(p) >= 0) return false;                             // already tiled
-    const int64_t tm = f16 ? kBM : kFM, tn = f16 ? kBN : kFN, tk = 64;
-    ps.m = (p->m + tm - 1) / tm * tm;
-    ps.n = (p->n + tn - 1) / tn * tn;
-    ps.k = (p->k + tk - 1) / tk * tk;
-    ps.es = f16 ? 2 : 4;
-    // A few rows or columns, padded 4 times or more in that direction alone:
-    // the general kernel fits its tiles to them (f16 64x4096x4096: 15 us
-    // against 88 us padded; 16x4096x4096: 12.5 us; f32 16x4096x4096: 17 us
-    // against 98 us).
-    if (ps.m >= 4 * p->m || ps.n >= 4 * p->n) return false;
-    if (ps.m >= (int64_t{1} << 31) || ps.n >= (int64_t{1} << 31) || ps.k >= (int64_t{1} << 31)) return false;
-    // Padded when the product is large (2^30 flop and up) or the padding at
-    // most 8 times the work.
+    if (mfmaForm(p) >= 0) return false;                             // whole blocks
+    if (p->m >= (1 << 30) || p->n >= (1 << 30) || p->k >= (1 << 30)) return false;
+    const int64_t tile = f16 ? kBM : kFM;
+    const int64_t pm = (p->m + tile - 1) / tile * tile, pn = (p->n + tile - 1) / tile * tile, pk = (p->k + 63) / 64 * 64;
+    // A few rows or columns, a quarter of a tile or less: the general kernel
+    // fits its tiles to them (f16 64x4096x4096: 15 us; f32 16x4096x4096: 17 us).
+    if (pm >= 4 * p->m || pn >= 4 * p->n) return false;
+    // Few tiles with a long K: a tile's K loop is serial, and the general
+    // kernel cuts K over waves and workgroups (f16 500^3: 5.8 against 11.8 us,
+    // 100x4096x4096: 18 against 40 us; f32 500^3: 6.7 against 13.0 us,
+    // 200x2000x2000: 29 against 40 us).
+    if (f16 && (p->m + kRM - 1) / kRM * ((p->n + kRN - 1) / kRN) < 64 && p->k >= 256) return false;
+    if (f32 && pm / kFM * (pn / kFN) <= 128 && p->k >= 128) return false;
     const double work = static_cast<double>(p->m) * static_cast<double>(p->n) * static_cast<double>(p->k);
-    const double padded = static_cast<double>(ps.m) * static_cast<double>(ps.n) * static_cast<double>(ps.k);
-    return 2.0 * work >= static_cast<double>(int64_t{1} << 30) || padded <= 8.0 * work;
+    return 2.0 * work >= static_cast<double>(int64_t{1} << 30) ||
+           static_cast<double>(pm) * static_cast<double>(pn) * static_cast<double>(pk) <= 8.0 * work;
 }
 
 size_t align256g(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 
-size_t padBytes(const PadShape& ps) {
-    return align256g(static_cast<size_t>(ps.m * ps.k) * ps.es) + align256g(static_cast<size_t>(ps.k * ps.n) * ps.es) +
-           align256g(static_cast<size_t>(ps.m * ps.n) * sizeof(float));
-}
-
-/// The padded launch's MFMA parameters, with A', B', C' carved from the
-/// workspace; false when the workspace is missing or too small.
-bool paddedParams(const mlkd_gemm* p, mlkd_gemm& q, PadShape& ps) {
-    if (p->work == nullptr || !padShape(p, ps) || p->work_bytes < static_cast<int64_t>(padBytes(ps))) return false;
-    unsigned char* w = static_cast<unsigned char*>(p->work);
-    q = *p;
-    q.a = w;
-    q.b = w + align256g(static_cast<size_t>(ps.m * ps.k) * ps.es);
-    q.c = static_cast<unsigned char*>(const_cast<void*>(q.b)) + align256g(static_cast<size_t>(ps.k * ps.n) * ps.es);
-    q.m = ps.m;
-    q.n = ps.n;
-    q.k = ps.k;
-    q.lda = ps.k;
-    q.ldb = ps.n;
-    q.ldc = ps.n;
-    q.work = nullptr;
-    q.work_bytes = 0;
-    return mfmaForm(&q) >= 0;
-}
-
-/// padBlock in 16-byte pieces, for source rows that start 16-byte aligned
-/// (src and lds * sizeof(T) multiples of 16; dcols a multiple of 16 /
-/// sizeof(T)). A piece that straddles `cols` is copied element by element.
+/// One operand's copy for a ragged member: rows x cols elements at stride ld
+/// into rows of dcols (whole 16-byte pieces), zeros past cols.
 template <typename T>
-__global__ __launch_bounds__(256) void padBlock16(const T* __restrict__ src, int64_t rows, int64_t cols,
-                                                  int64_t lds, T* __restrict__ dst, int64_t drows, int64_t dcols) {
+struct RowCopy {
+    const T* src;
+    T* dst;
+    int64_t rows, cols, ld, dcols;
+};
+
+/// Both operands' copies in one launch (blockIdx.z), in 16-byte pieces read at
+/// any element alignment; the piece that straddles `cols` element by element.
+template <typename T>
+__global__ __launch_bounds__(256) void copyRows(RowCopy<T> first, RowCopy<T> second) {
+    const RowCopy<T>& c = blockIdx.z == 0 ? first : second;
     constexpr int V = 16 / sizeof(T);
-    const int64_t pieces = dcols / V;
-    for (int64_t r = blockIdx.y; r < drows; r += gridDim.y) {
+    struct __attribute__((packed, aligned(sizeof(T)))) Any16 {
+        u32x4 v;
+    };
+    const int64_t pieces = c.dcols / V;
+    for (int64_t r = blockIdx.y; r < c.rows; r += gridDim.y) {
         for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < pieces;
              j += static_cast<int64_t>(gridDim.x) * 256) {
             const int64_t c0 = j * V;
+            const T* src = c.src + r * c.ld + c0;
             u32x4 v = {0u, 0u, 0u, 0u};
-            if (r < rows && c0 + V <= cols) {
-                v = *reinterpret_cast<const u32x4*>(src + r * lds + c0);
-            } else if (r < rows && c0 < cols) {
+            if (c0 + V <= c.cols) {
+                v = reinterpret_cast<const Any16*>(src)->v;
+            } else if (c0 < c.cols) {
                 T e[V];
 #pragma unroll
-                for (int i = 0; i < V; ++i) e[i] = c0 + i < cols ? src[r * lds + c0 + i] : T(0);
+                for (int i = 0; i < V; ++i) e[i] = c0 + i < c.cols ? src[i] : T{0};
                 v = __builtin_bit_cast(u32x4, e);
             }
-            *reinterpret_cast<u32x4*>(dst + r * dcols + c0) = v;
+            *reinterpret_cast<u32x4*>(c.dst + r * c.dcols + c0) = v;
         }
     }
 }
 
-/// unpadBlock in 16-byte pieces (dst and ldd * 4 multiples of 16 bytes); a
-/// piece that straddles `cols` is copied element by element.
-__global__ __launch_bounds__(256) void unpadBlock16(const uint32_t* __restrict__ src, int64_t scols,
-                                                    uint32_t* __restrict__ dst, int64_t rows, int64_t cols,
-                                                    int64_t ldd) {
-    const int64_t pieces = (cols + 3) / 4;
-    for (int64_t r = blockIdx.y; r < rows; r += gridDim.y) {
-        for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < pieces;
-             j += static_cast<int64_t>(gridDim.x) * 256) {
-            const int64_t c0 = j * 4;
-            if (c0 + 4 <= cols) {
-                *reinterpret_cast<u32x4*>(dst + r * ldd + c0) = *reinterpret_cast<const u32x4*>(src + r * scols + c0);
-            } else {
-                for (int64_t c = c0; c < cols; ++c) dst[r * ldd + c] = src[r * scols + c];
-            }
-        }
-    }
+/// How such a product runs: an operand off 16 bytes, or with rows that are, is
+/// copied to aligned rows first.
+struct RaggedPlan {
+    bool copyA, copyB;
+    bool wide;        // f16 tiles of 256 x 256, not 128 x 128
+    int64_t ka, nb;   // columns of A's and B's rows as the kernel reads them
+    size_t bytesA, bytesB;
+};
+
+bool raggedPlan(const mlkd_gemm* p, RaggedPlan& r) {
+    if (!raggedShape(p) || (reinterpret_cast<uintptr_t>(p->c) & 3) != 0) return false;
+    const int64_t es = p->a_dtype == MLKD_F16 ? 2 : 4, v = 16 / es;
+    r.copyA = p->k % v != 0 || p->lda % v != 0 || !aligned16(p->a);
+    r.copyB = p->n % v != 0 || p->ldb % v != 0 || !aligned16(p->b);
+    // The tile with the shorter run: rounds over 256 CUs of K steps of 32, each
+    // 0.31 us on 128 x 128 and 0.65-0.85 on 256 x 256, and the start and end
+    // (2000^3: 25 us against 50, 3000^3: 93 against 71, 4000^3: 160 against 119).
+    const auto run = [&](int64_t t, double step, double ends) {
+        const int64_t tiles = (p->m + t - 1) / t * ((p->n + t - 1) / t);
+        return static_cast<double>((tiles + 255) / 256) * static_cast<double>((p->k + 31) / 32) * step + ends;
+    };
+    r.wide = es == 2 && run(256, 0.75, 10.0) < run(128, 0.31, 5.0);
+    r.ka = r.copyA ? (p->k + v - 1) / v * v : p->k;
+    r.nb = r.copyB ? (p->n + v - 1) / v * v : p->n;
+    r.bytesA = r.copyA ? align256g(static_cast<size_t>(p->m * r.ka * es)) : 0;
+    r.bytesB = r.copyB ? align256g(static_cast<size_t>(p->k * r.nb * es)) : 0;
+    // Lane offsets of 32 bits (f16).
+    const int64_t lda = r.copyA ? r.ka : p->lda, ldb = r.copyB ? r.nb : p->ldb;
+    return es == 4 || (lda < (int64_t{1} << 23) && ldb < (int64_t{1} << 25));
 }
 
-template <typename T>
-void launchPad(const void* src, int64_t rows, int64_t cols, int64_t lds, void* dst, int64_t drows, int64_t dcols,
-               hipStream_t st) {
-    constexpr int V = 16 / sizeof(T);
-    const unsigned gy = static_cast<unsigned>(std::min<int64_t>(drows, 4096));
-    if ((reinterpret_cast<uintptr_t>(src) & 15) == 0 && (lds * static_cast<int64_t>(sizeof(T))) % 16 == 0 &&
-        dcols % V == 0) {
-        const unsigned gx = static_cast<unsigned>(std::min<int64_t>((dcols / V + 255) / 256, 64));
-        hipLaunchKernelGGL(padBlock16<T>, dim3(gx, gy), dim3(256), 0, st, static_cast<const T*>(src), rows, cols, lds,
-                           static_cast<T*>(dst), drows, dcols);
-        return;
-    }
-    const unsigned gx = static_cast<unsigned>(std::min<int64_t>((dcols + 255) / 256, 64));
-    hipLaunchKernelGGL(padBlock<T>, dim3(gx, gy), dim3(256), 0, st, static_cast<const T*>(src), rows, cols, lds,
-                       static_cast<T*>(dst), drows, dcols);
+/// Whether the copies, if any, have their workspace.
+bool roomFor(const mlkd_gemm* p, const RaggedPlan& r) {
+    const int64_t need = static_cast<int64_t>(r.bytesA + r.bytesB);
+    return need == 0 || (p->work != nullptr && p->work_bytes >= need);
 }
 
-int launchPadded(const mlkd_gemm* p, const mlkd_gemm& q, const PadShape& ps, hipStream_t st) {
-    if (ps.es == 2) {
-        launchPad<uint16_t>(p->a, p->m, p->k, p->lda, const_cast<void*>(q.a), ps.m, ps.k, st);
-        launchPad<uint16_t>(p->b, p->k, p->n, p->ldb, const_cast<void*>(q.b), ps.k, ps.n, st);
-    } else {
-        launchPad<uint32_t>(p->a, p->m, p->k, p->lda, const_cast<void*>(q.a), ps.m, ps.k, st);
-        launchPad<uint32_t>(p->b, p->k, p->n, p->ldb, const_cast<void*>(q.b), ps.k, ps.n, st);
+template <typename Args, typename T>
+Args raggedArgs(const mlkd_gemm* p, const RaggedPlan& r, int tileM, int tileN, hipStream_t st) {
+    using Bits = std::conditional_t<sizeof(T) == 2, uint16_t, uint32_t>;
+    unsigned char* w = static_cast<unsigned char*>(p->work);
+    Args q;
+    q.a = r.copyA ? reinterpret_cast<const T*>(w) : static_cast<const T*>(p->a);
+    q.b = r.copyB ? reinterpret_cast<const T*>(w + r.bytesA) : static_cast<const T*>(p->b);
+    q.c = static_cast<float*>(p->c);
+    q.m = static_cast<int>(p->m);
+    q.n = static_cast<int>(p->n);
+    q.k = static_cast<int>(p->k);
+    q.ka = static_cast<int>(r.ka);
+    q.nb = static_cast<int>(r.nb);
+    q.tilesM = (q.m + tileM - 1) / tileM;
+    q.tilesN = (q.n + tileN - 1) / tileN;
+    q.lda = r.copyA ? r.ka : p->lda;
+    q.ldb = r.copyB ? r.nb : p->ldb;
+    q.ldc = p->ldc;
+    q.skip = p->skip_zero_a != 0 ? 1 : 0;
+    if (r.copyA || r.copyB) {
+        const RowCopy<Bits> a = {static_cast<const Bits*>(p->a), reinterpret_cast<Bits*>(w), p->m, p->k, p->lda, r.ka};
+        const RowCopy<Bits> b = {static_cast<const Bits*>(p->b), reinterpret_cast<Bits*>(w + r.bytesA), p->k, p->n,
+                                 p->ldb, r.nb};
+        const int64_t v = 16 / static_cast<int64_t>(sizeof(T));
+        const int64_t rows = std::max(r.copyA ? p->m : 0, r.copyB ? p->k : 0);
+        const int64_t pieces = std::max(r.copyA ? r.ka / v : 0, r.copyB ? r.nb / v : 0);
+        const dim3 grid(static_cast<unsigned>(std::min<int64_t>((pieces + 255) / 256, 64)),
+                        static_cast<unsigned>(std::min<int64_t>(rows, 4096)), r.copyA && r.copyB ? 2 : 1);
+        hipLaunchKernelGGL(copyRows<Bits>, grid, dim3(256), 0, st, r.copyA ? a : b, b);
     }
-    // C += A*B reads C: its padded copy starts from C (and zeros).
-    if (p->accumulate != 0) launchPad<uint32_t>(p->c, p->m, p->n, p->ldc, q.c, ps.m, ps.n, st);
-    if (hipGetLastError() != hipSuccess) return MLKD_RT_LAUNCH;
-    if (const int rc = launchMfma(&q, mfmaForm(&q), st); rc != 0) return rc;
-    const unsigned gy = static_cast<unsigned>(std::min<int64_t>(p->m, 4096));
-    if ((reinterpret_cast<uintptr_t>(p->c) & 15) == 0 && p->ldc % 4 == 0) {
-        const unsigned gx = static_cast<unsigned>(std::min<int64_t>(((p->n + 3) / 4 + 255) / 256, 64));
-        hipLaunchKernelGGL(unpadBlock16, dim3(gx, gy), dim3(256), 0, st, static_cast<const uint32_t*>(q.c), ps.n,
-                           static_cast<uint32_t*>(p->c), p->m, p->n, p->ldc);
+    return q;
+}
+
+int launchRagged(const mlkd_gemm* p, const RaggedPlan& r, hipStream_t st) {
+    if (raiseLdsLimits() != 0) return MLKD_RT_LAUNCH;
+    const bool acc = p->accumulate != 0;
+    if (p->a_dtype == MLKD_F32) {
+        const RaggedF32 q = raggedArgs<RaggedF32, float>(p, r, kFM, kFN, st);
+        hipLaunchKernelGGL((acc ? RaggedDma{gemmF32Dma<true>} : RaggedDma{gemmF32Dma<false>}),
+                           dim3(static_cast<unsigned>(q.tilesM * q.tilesN)), dim3(512), kLdsF32Dma, st, q);
+    } else if (r.wide) {
+        const RaggedF16Wide q = raggedArgs<RaggedF16Wide, _Float16>(p, r, kBM, kBN, st);
+        hipLaunchKernelGGL((acc ? RaggedWide8s{gemmF16Dma8s<true>} : RaggedWide8s{gemmF16Dma8s<false>}),
+                           dim3(static_cast<unsigned>(q.tilesM * q.tilesN)), dim3(512), kLdsDma, st, q);
     } else {
-        const unsigned gx = static_cast<unsigned>(std::min<int64_t>((p->n + 255) / 256, 64));
-        hipLaunchKernelGGL(unpadBlock<uint32_t>, dim3(gx, gy), dim3(256), 0, st, static_cast<const uint32_t*>(q.c),
-                           ps.n, static_cast<uint32_t*>(p->c), p->m, p->n, p->ldc);
+        const RaggedF16 q = raggedArgs<RaggedF16, _Float16>(p, r, kRM, kRN, st);
+        hipLaunchKernelGGL((acc ? Ragged8s{gemmF16Dma8s<true>} : Ragged8s{gemmF16Dma8s<false>}),
+                           dim3(static_cast<unsigned>(q.tilesM * q.tilesN)), dim3(256), kLdsRagged, st, q);
     }
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
 }
@@ -1958,18 +2355,21 @@ int launchPadded(const mlkd_gemm* p, const mlkd_gemm& q, const PadShape& ps, hip
 extern "C" void mlkd_gemm_set_variant(int variant) { gGemmF16Variant = variant; }
 
 extern "C" int64_t mlkd_gemm_pad_bytes(const mlkd_gemm* p) {
-    PadShape ps;
-    if (p == nullptr) return 0;
-    if (padShape(p, ps)) return static_cast<int64_t>(padBytes(ps));
-    return tiled(p) ? 0 : mlkdGemmGeneralBytes(p);
+    if (p == nullptr || tiled(p)) return 0;
+    RaggedPlan r;
+    return raggedPlan(p, r) ? static_cast<int64_t>(r.bytesA + r.bytesB) : mlkdGemmGeneralBytes(p);
+}
+
+extern "C" void mlkd_gemm_tile(const mlkd_gemm* p, int64_t* rows, int64_t* cols) {
+    RaggedPlan r;
+    if (!raggedPlan(p, r)) return mlkdGemmGeneralTile(p, rows, cols);
+    *rows = *cols = p->a_dtype == MLKD_F32 ? kFM : (r.wide ? kBM : kRM);
 }
 
 extern "C" const char* mlkd_gemm_kernel_name(const mlkd_gemm* p) {
-    {
-        // A padded launch is named by the MFMA form it runs.
-        mlkd_gemm q;
-        PadShape ps;
-        if (paddedParams(p, q, ps)) return mlkd_gemm_kernel_name(&q);
+    if (RaggedPlan r; raggedPlan(p, r) && roomFor(p, r)) {
+        if (p->a_dtype == MLKD_F32) return p->accumulate != 0 ? "gemmF32Dma<true>" : "gemmF32Dma<false>";
+        return p->accumulate != 0 ? "gemmF16Dma8s<true>" : "gemmF16Dma8s<false>";
     }
     const bool acc = p->accumulate != 0;
     switch (p->skip_zero_a != 0 && !acc ? -1 : mfmaForm(p)) {
@@ -1998,13 +2398,6 @@ extern "C" int mlkd_launch_gemm(const mlkd_gemm* p, void* stream) {
     // accumulators met an infinity or a NaN recomputes its block exactly. One
     // launch, no scratch, no host read-back.
     if (tiled(p)) return launchMfma(p, mfmaForm(p), st);
-    {
-        mlkd_gemm q;
-        PadShape ps;
-        if (paddedParams(p, q, ps)) {
-            if (raiseLdsLimits() != 0) return MLKD_RT_LAUNCH;
-            return launchPadded(p, q, ps, st);
-        }
-    }
+    if (RaggedPlan r; raggedPlan(p, r) && roomFor(p, r)) return launchRagged(p, r, st);
     return mlkdLaunchGemmGeneral(p, st);
 }

@@ -15,3 +15,6 @@ int64_t mlkdGemmGeneralBytes(const mlkd_gemm* p);
 /// The kernels a launch runs, joined by '+', as mlkd_gemm_kernel_name names
 /// them (p->work as the launch will have it).
 const char* mlkdGemmGeneralName(const mlkd_gemm* p);
+
+/// The output tile of a workgroup of that launch.
+void mlkdGemmGeneralTile(const mlkd_gemm* p, int64_t* rows, int64_t* cols);

@@ -442,7 +442,7 @@ DirectPlan directPlan(const mlkd_gemm* p) {
     const int v = f16 ? 8 : (f32 ? 4 : 2), ks = 4 * v;
     const uintptr_t es = 16u / static_cast<uintptr_t>(v), os = f64 ? 8 : 4;
     if (p->m <= 0 || p->n < v || p->k < ks || p->m >= (1 << 30) || p->n >= (1 << 30) || p->k >= (1 << 30) ||
-        p->lda >= (1 << 22) || p->ldb >= (1 << 22) || reinterpret_cast<uintptr_t>(p->a) % es != 0 ||
+        p->lda >= (1 << 26) / static_cast<int64_t>(es) || p->ldb >= (1 << 26) || reinterpret_cast<uintptr_t>(p->a) % es != 0 ||
         reinterpret_cast<uintptr_t>(p->b) % es != 0 || reinterpret_cast<uintptr_t>(p->c) % os != 0) {
         return d;
     }
@@ -546,17 +546,10 @@ int64_t partBytes(const mlkd_gemm* p, const DirectPlan& d) {
 
 }  // namespace
 
-extern "C" int mlkd_gemm_general_tile(const mlkd_gemm* p, int64_t* rows, int64_t* cols, int64_t* workgroups) {
+void mlkdGemmGeneralTile(const mlkd_gemm* p, int64_t* rows, int64_t* cols) {
     const DirectPlan d = directPlan(p);
-    if (d.mt == 0) {
-        *rows = *cols = 64;
-        *workgroups = ((p->m + 63) / 64) * ((p->n + 63) / 64);
-        return 0;
-    }
-    *rows = 16 * d.mt;
-    *cols = 16 * (p->a_dtype == MLKD_F16 ? 8 : (p->a_dtype == MLKD_F32 ? 4 : 2));
-    *workgroups = static_cast<int64_t>(d.tilesM) * d.tilesN;
-    return d.ranges;
+    *rows = d.mt == 0 ? 64 : 16 * d.mt;
+    *cols = d.mt == 0 ? 64 : 16 * (p->a_dtype == MLKD_F16 ? 8 : (p->a_dtype == MLKD_F32 ? 4 : 2));
 }
 
 const char* mlkdGemmGeneralName(const mlkd_gemm* p) {

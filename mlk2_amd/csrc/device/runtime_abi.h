@@ -88,14 +88,12 @@ int mlkd_launch_softmax(const mlkd_softmax* p, void* stream);
 /// with plain stores; waves <= 0 keeps the default grid).
 void mlkd_softmax_set_variant(int variant, int64_t waves);
 int mlkd_launch_gemm(const mlkd_gemm* p, void* stream);
-/// Bytes of workspace that let mlkd_launch_gemm run `p` on an MFMA form
-/// through zero-padded copies of A, B and C, or the general kernel on several
-/// K ranges; 0 when the shape needs none.
+/// Bytes of workspace for mlkd_launch_gemm's aligned copies of A and B (a
+/// ragged MFMA member), or for the sums of the general kernel's K ranges; 0
+/// when `p` needs none.
 int64_t mlkd_gemm_pad_bytes(const mlkd_gemm* p);
-/// The general kernel's output tile and workgroups (per K range) for `p`'s
-/// shape; returns the K ranges it is cut into given workspace (0: the scalar
-/// kernel).
-int mlkd_gemm_general_tile(const mlkd_gemm* p, int64_t* rows, int64_t* cols, int64_t* workgroups);
+/// The output tile of a workgroup for a shape no whole-block form tiles.
+void mlkd_gemm_tile(const mlkd_gemm* p, int64_t* rows, int64_t* cols);
 /// The symbol of the kernel mlkd_launch_gemm runs for `p` (the MFMA form, or
 /// the general kernel), as profilers print it without the parameters. A
 /// skip-zero-A launch is the same single kernel.

@@ -50,11 +50,11 @@ typedef struct mlkd_gemm {
        its block exactly. Otherwise the general kernel runs everything. */
     int32_t skip_zero_a;
     int32_t pad_;
-    /* Device workspace for shapes the MFMA forms do not tile
-       (mlkd_gemm_pad_bytes): the operands are copied into zero-padded
-       blocks there, the MFMA form runs on them and C is copied back; or the
-       general kernel's K ranges leave their sums there. NULL (or too small)
-       runs such shapes on the general kernel in one range. */
+    /* Device workspace for shapes the MFMA forms do not tile in whole blocks
+       (mlkd_gemm_pad_bytes): operands whose rows are off 16 bytes are copied
+       to aligned ones there, or the general kernel's K ranges leave their
+       sums there. NULL (or too small) runs such shapes on the general kernel
+       in one range. */
     void* work;
     int64_t work_bytes;
 } mlkd_gemm;

@@ -346,7 +346,7 @@ const char* HipLoadedKernel::stepKernelName(size_t si) const {
             mlkd_gemm p;
             fillGemmParams(st, ptr, p);
             if (const int64_t need = mlkd_gemm_pad_bytes(&p); need > 0) {
-                p.work = ptr[0];   // runDevice gives such a step its padding workspace
+                p.work = ptr[0];   // runDevice gives such a step its workspace
                 p.work_bytes = need;
             }
             name = mlkd_gemm_kernel_name(&p);
@@ -358,7 +358,7 @@ const char* HipLoadedKernel::stepKernelName(size_t si) const {
                 p.scratch_bytes = need;
             }
             if (const int64_t need = mlkd_score_pad_bytes(&p); need > 0) {
-                p.work = ptr[0];   // runDevice gives such a step its padding workspace
+                p.work = ptr[0];   // runDevice gives such a step its workspace
                 p.work_bytes = need;
             }
             name = mlkd_score_kernel_names(&p);
@@ -438,9 +438,10 @@ int HipLoadedKernel::arenaLayout(const DeviceBinding* binds, int64_t elements, c
               std::to_string(arena.bytes);
         return MLKHIP_REFUSED;
     }
-    // Padding workspaces (GEMM shapes off the MFMA tiles, score-softmax
-    // lengths off the two-pass blocks) take the room that is left, in step
-    // order; a step whose workspace does not fit runs on the general kernels.
+    // Workspaces a step can do without (GEMM shapes off the MFMA tiles,
+    // score-softmax lengths off the two-pass blocks) take the room that is
+    // left, in step order; a step whose workspace does not fit runs on the
+    // general kernels.
     padOff.assign(plan_.steps.size(), SIZE_MAX);
     for (size_t si = 0; si < plan_.steps.size(); ++si) {
         const Step& st = plan_.steps[si];
@@ -596,10 +597,11 @@ int HipLoadedKernel::runDevice(const DeviceBinding* binds, int n, const double* 
                 // products whose skip changes C beyond the sign of a zero
                 // sum) is taken inside the MFMA kernel, per wave: one launch,
                 // no host read-back.
-                // A shape the MFMA forms do not tile runs on zero-padded
-                // copies in a per-stream workspace, or, for the
-                // allocation-free entry, in the arena when they fit there
-                // (else on the general kernel).
+                // Operands with unaligned rows are copied to aligned ones, and
+                // the general kernel's K ranges leave their sums, in a
+                // per-stream workspace, or, for the allocation-free entry, in
+                // the arena when they fit there (else the general kernel
+                // runs, in one range).
                 const int64_t need = mlkd_gemm_pad_bytes(&p);
                 if (need > 0 && arena != nullptr && padOff[si] != SIZE_MAX) {
                     p.work = arena->base + padOff[si];

@@ -362,9 +362,8 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
         case StepKind::Gemm: {
             // f16 x f16 -> f32 with M, N % 256 and K % 64 runs the MFMA forms
             // on 256 x 256 tiles (forms 5 and 6: 128 x 256); f32 with M, N % 64
-            // and K % 32 the 64 x 64 MFMA tiles (on padded copies where
-            // that pays); anything else the bounds-checked general kernel,
-            // on tiles it fits to the shape.
+            // and K % 32 the 64 x 64 MFMA tiles; anything else a
+            // bounds-checked kernel on tiles fitted to the shape.
             instances = st.m * st.n;
             auto dt = [&](uint32_t b) { return km.buffers[b].dtype; };
             const bool f16 = dt(st.a) == Dtype::F16 && dt(st.b) == Dtype::F16 && dt(st.c) == Dtype::F32 &&
@@ -394,7 +393,8 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
                 p.ldc = st.ldc;
                 p.variant = -1;
                 int64_t rows = 0, cols = 0;
-                mlkd_gemm_general_tile(&p, &rows, &cols, &workgroups);
+                mlkd_gemm_tile(&p, &rows, &cols);
+                workgroups = ((st.m + rows - 1) / rows) * ((st.n + cols - 1) / cols);
                 perGroup = rows * cols;
                 covered = workgroups * perGroup >= instances;
                 form = "output tiles fitted to the shape, bounds-checked";
