@@ -88,6 +88,27 @@ int mlkd_rt_malloc(void** p, size_t bytes) {
     return mapErr(hipMalloc(p, bytes), MLKD_RT_ALLOC);
 }
 
+int mlkd_rt_malloc_spare(void** p, size_t bytes, void* stream) {
+    *p = nullptr;
+    // An allocation would end a capture of this stream; a relaxed thread may
+    // allocate beside a capture of another.
+    hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
+        (void)hipGetLastError();
+        return MLKD_RT_ALLOC;
+    }
+    if (status != hipStreamCaptureStatusNone) return MLKD_RT_ALLOC;
+    hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
+    if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
+        (void)hipGetLastError();
+        return MLKD_RT_ALLOC;
+    }
+    const int rc = mlkd_rt_malloc(p, bytes);
+    if (rc != 0) (void)hipGetLastError();
+    (void)hipThreadExchangeStreamCaptureMode(&mode);
+    return rc;
+}
+
 int mlkd_rt_free(void* p) {
     if (p == nullptr) return 0;
     return mapErr(hipFree(p), MLKD_RT_ALLOC);

@@ -26,6 +26,9 @@ int mlkd_rt_device_arch(int dev, char* buf, size_t cap);
 int mlkd_rt_device_info(int dev, int* cu_count, int64_t* max_grid_x, int* max_block,
                         int64_t* global_mem);
 int mlkd_rt_malloc(void** p, size_t bytes);
+/// mlkd_rt_malloc for memory the caller can do without: fails while `stream`
+/// is being captured and leaves a capture elsewhere in the process alone.
+int mlkd_rt_malloc_spare(void** p, size_t bytes, void* stream);
 int mlkd_rt_free(void* p);
 /// Page-locked host memory (hipHostMalloc): copies between it and the device
 /// run at DMA rate. Released by mlkd_rt_host_free.
@@ -103,8 +106,10 @@ const char* mlkd_softmax_kernel_name(const mlkd_softmax* p);
 /// Likewise for score-softmax: its kernels joined by '+' (valid until this
 /// thread's next call).
 const char* mlkd_score_kernel_names(const mlkd_score_softmax* p);
-/// Workspace bytes that let mlkd_launch_score_softmax run a sequence length
-/// off the two-pass form's blocks on zero-padded copies; 0 when none applies.
+/// Workspace bytes (16-byte aligned) that let mlkd_launch_score_softmax take
+/// the two-pass form where it is not given scratch for it (head dim 64,
+/// sequences off whole pairs of 128-key panels, those off the panels on
+/// zero-padded copies), or split the keys further; 0 when none applies.
 int64_t mlkd_score_pad_bytes(const mlkd_score_softmax* p);
 /// Process default of the f16 GEMM launch form (8: direct-to-LDS ring with 8
 /// waves of 16x16x32 tiles, the default; 7: the same ring with 4 waves of
@@ -112,9 +117,13 @@ int64_t mlkd_score_pad_bytes(const mlkd_score_softmax* p);
 /// 3: pipelined step; 5/6: 128x256 tiles, two workgroups per CU).
 void mlkd_gemm_set_variant(int variant);
 int mlkd_launch_score_softmax(const mlkd_score_softmax* p, void* stream);
-/// Scratch bytes the two-pass score-softmax form needs for `p`'s shape (0 when
-/// that form does not apply).
+/// Scratch bytes the two-pass score-softmax form is always given for `p`'s
+/// shape (0 when it is not).
 int64_t mlkd_score_scratch_bytes(const mlkd_score_softmax* p);
+/// Key ranges per 128-row block of that form on a workspace of
+/// mlkd_score_pad_bytes (its sequence length rounded up to 128); 0 for a shape
+/// it does not take.
+int mlkd_score_ranges(const mlkd_score_softmax* p);
 /// Variant-space hook for score-softmax (0: best form for the shape, 1: scores
 /// then softmax, 2: fused single pass, 3: two-pass 256 x 256 blocks, 8:
 /// two-pass query-stationary).

@@ -5,8 +5,8 @@
 //
 // The output write (4 * batch * seq^2 bytes) bounds the class; the scores are
 // a GEMM with K = dim on v_mfma_f32_32x32x16_f16. Forms, best first:
-//   * two-pass, query-stationary (dim 128, seq % 256 == 0, seq <= 8192): a
-//     statistics pass and a recompute-and-write pass (scoreStatsQ /
+//   * two-pass, query-stationary (dim 128, or 64 from 512 keys, seq % 128 == 0,
+//     seq <= 8192): a statistics pass and a recompute-and-write pass (scoreStatsQ /
 //     scoreStoreQ), rows' partial statistics in artifact scratch;
 //   * scores, then the softmax kernel in place over S (any shape, f16);
 //   * a scalar f64 path for other dtypes.
@@ -67,66 +67,88 @@ __global__ __launch_bounds__(256) void scoresF16(const _Float16* __restrict__ Q,
 }
 
 // ------------------------------------------------------------ two pass ----
-constexpr int kD2 = 128;                 // head dim
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
-// Query-stationary form of the two passes (dim 128, seq a multiple of 256).
-// A wave owns 32 query rows and holds their Q fragments in registers for the
-// whole kernel; a workgroup of 4 waves (128 rows) streams one half of the
-// batch's keys through LDS in 128-key panels, double buffered, the next
-// panel's global loads in flight during the current panel's MFMAs. 73 KiB
-// of LDS and <= 256 registers per lane let two workgroups share a CU.
+// Query-stationary form of the two passes (head dim D 64 or 128, seq a
+// multiple of 128). A wave owns 32 query rows and holds their Q fragments in
+// registers for the whole kernel; a workgroup of 4 waves (128 rows) streams one
+// of NR ranges of the batch's keys through LDS in 128-key panels, double
+// buffered, the next panel's global loads in flight during the current panel's
+// MFMAs. At most 73 KiB of LDS and 256 registers per lane let two workgroups
+// share a CU. Scores by 64 x 128 tiles and a softmax over S in place read S
+// back and each K element once per 64 rows: at D 64, 8 x 1024 took 23.5 us
+// and takes 14.4, 16 x 2048 165 and 67.
 //   Pass 1 (scoreStatsQ) computes D = K Q^T per panel, so each lane holds 64
 //   of its query's scores per panel and keeps a running max and
 //   sum(exp(v - max)) in two registers; the lane 32 away holds the other
 //   keys of the same query, and the pair is combined once at the end into
-//   scratch[row][key half].
+//   scratch[row][key range].
 //   Pass 2 (scoreStoreQ) computes D = Q K^T per panel and writes
-//   exp2(v - (max + log2 sum)) for the panel at once: each 32-lane half-wave
-//   stores one 128-byte line, while the other workgroup on the CU computes.
+//   softmax of the panel at once: each 32-lane half-wave stores
+//   one 128-byte line, while the other workgroup on the CU computes.
 // Both passes work in base 2 with log2(e) folded into 1/div and the bias, so
-// a score costs one fused multiply-add and one v_exp_f32. Pass 2 is bound by
-// its stores (256 MiB in the MFMA output layout); pass 1 by its MFMAs and
-// the VALU work per score together.
+// a score costs one fused multiply-add and one v_exp_f32. 16 x 2048 x 128: pass
+// 1 takes 29 us, bound by its v_exp_f32 (13 us) and MFMAs (7 us), which the
+// two waves of a SIMD overlap in part (panels of 64 keys and four workgroups a
+// CU: no faster); pass 2 takes 45-48 us, bound by its 256 MiB of stores.
 constexpr int kPanelQ = 128;                   // keys per streamed panel
+constexpr int kMaxRangesQ = 8;                 // key ranges per 128-row block
 constexpr float kLog2e = 1.44269504088896340736f;
-constexpr int kRowQ = kD2 + 8;                 // halves per LDS panel row
-constexpr int kPanelHalvesQ = kPanelQ * kRowQ;
-constexpr size_t kLdsStoreQ = 2 * kPanelHalvesQ * sizeof(_Float16);  // pass 1 adds seq/2 floats of bias
-constexpr int64_t kMaxSeqQ = 8192;             // pass 1's LDS stays <= 86 KiB
+template <int D>
+constexpr int kRowQ = D + 8;                   // halves per LDS panel row
+template <int D>
+constexpr int kPanelHalvesQ = kPanelQ * kRowQ<D>;
+template <int D>
+constexpr size_t kLdsStoreQ = 2 * kPanelHalvesQ<D> * sizeof(_Float16);  // pass 1 adds its keys' bias
+constexpr int64_t kMaxSeqQ = 8192;             // pass 1's LDS stays <= 100 KiB
 
 /// The max to subtract before exp2: a max of -inf (every score so far -inf)
 /// is replaced by 0, so those scores contribute exp2(-inf) = 0 rather than
 /// exp2(-inf - -inf) = NaN; the stored max stays -inf.
 __device__ __forceinline__ float finiteOr0(float m) { return m == -INFINITY ? 0.0f : m; }
 
-/// 256 threads: global -> registers for one 128-key panel (8 chunks each).
-__device__ __forceinline__ void loadPanelQ(const _Float16* __restrict__ k, int tid, u32x4v (&v)[8]) {
+/// The bias in base 2. A finite one stays finite, so that keys masked with the
+/// lowest float still share a row that has no others.
+__device__ __forceinline__ float biasLog2(float b) {
+    const float t = b * kLog2e;
+    return __builtin_isinf(t) && !__builtin_isinf(b) ? __builtin_copysignf(3.402823466e+38f, t) : t;
+}
+
+/// 256 threads: global -> registers for one 128-key panel (D / 16 16-byte
+/// pieces each), which is contiguous in K.
+template <int D>
+__device__ __forceinline__ void loadPanelQ(const _Float16* __restrict__ k, int tid, u32x4v (&v)[D / 16]) {
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int c = j * 256 + tid;
-        v[j] = *reinterpret_cast<const u32x4v*>(k + (c >> 4) * kD2 + (c & 15) * 8);
+    for (int j = 0; j < D / 16; ++j) v[j] = *reinterpret_cast<const u32x4v*>(k + (j * 256 + tid) * 8);
+}
+
+/// Registers -> LDS: key i of the panel to row i, or (QUADS) to row
+/// i % 4 * 32 + i / 4.
+template <int D, bool QUADS = false>
+__device__ __forceinline__ void storePanelQ(_Float16* dst, int tid, const u32x4v (&v)[D / 16]) {
+#pragma unroll
+    for (int j = 0; j < D / 16; ++j) {
+        const int c = j * 256 + tid, key = c / (D / 8);
+        const int row = QUADS ? (key & 3) * 32 + (key >> 2) : key;
+        *reinterpret_cast<u32x4v*>(dst + row * kRowQ<D> + c % (D / 8) * 8) = v[j];
     }
 }
 
-__device__ __forceinline__ void storePanelQ(_Float16* dst, int tid, const u32x4v (&v)[8]) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-        const int c = j * 256 + tid;
-        *reinterpret_cast<u32x4v*>(dst + (c >> 4) * kRowQ + (c & 15) * 8) = v[j];
-    }
-}
-
-/// Workgroup coordinates: batch, 128-row block, key half. A batch's
-/// workgroups are contiguous within one XCD's share of the grid.
-__device__ __forceinline__ void blockOfQ(int rowBlocks, int64_t& b, int& rb, int& kh) {
-    const int total = static_cast<int>(gridDim.x);
+/// Workgroup coordinates: batch, 128-row block, key range of nr, and the
+/// range's first key and length: `per` keys, the last range what is left. A
+/// batch's workgroups are contiguous within one XCD's share of the grid, a row
+/// block's side by side (ranges as the slow dimension: 16 x 2048 x 128 90.7
+/// against 77 us).
+__device__ __forceinline__ void blockOfQ(int seq, int nr, int per, int64_t& b, int& rb, int& kr, int& k0, int& keys) {
+    const int total = static_cast<int>(gridDim.x), panels = seq / kPanelQ;
     int id = static_cast<int>(blockIdx.x);
     if (total % 8 == 0) id = (id % 8) * (total / 8) + id / 8;
-    b = id / (rowBlocks * 2);
-    const int rem = id % (rowBlocks * 2);
-    rb = rem / 2;
-    kh = rem % 2;
+    kr = id % nr;
+    id /= nr;
+    b = id / panels;
+    rb = id % panels;
+    k0 = kr * per;
+    keys = min(per, seq - k0);
 }
 
 /// Pass-1 statistics of this wave's 32 queries of row block (b, rb) over
@@ -134,27 +156,29 @@ __device__ __forceinline__ void blockOfQ(int rowBlocks, int64_t& b, int& rb, int
 /// running max and sum(exp2(v - max)) of its query; the lane 32 away holds
 /// the other keys of the same query and the pair is combined at the end.
 /// Returns (max, sum) of query row `qrow` in base 2 (both half-waves agree).
+template <int D>
 __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                               const float* __restrict__ bias, int seq, float c2, int64_t b,
                                               int rb, int k0, int keys, _Float16* ldsQ, int64_t& qrow) {
-    float* lbias = reinterpret_cast<float*>(ldsQ + 2 * kPanelHalvesQ);  // this key range's bias
+    float* lbias = reinterpret_cast<float*>(ldsQ + 2 * kPanelHalvesQ<D>);  // this key range's bias
     const int tid = threadIdx.x;
     const int lane = tid & 63, wave = tid >> 6, l32 = lane & 31, hl = lane >> 5;
     const int np = keys / kPanelQ;
     qrow = b * seq + static_cast<int64_t>(rb) * 128 + wave * 32 + l32;
-    f16x8 xq[8];                                  // B operand: this lane's query, 8 x 16 head dims
+    constexpr int KS = D / 16;
+    f16x8 xq[KS];                                 // B operand: this lane's query, KS x 16 head dims
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) xq[ks] = *reinterpret_cast<const f16x8*>(Q + qrow * kD2 + ks * 16 + hl * 8);
-    for (int i = tid; i < keys; i += 256) lbias[i] = bias[k0 + i] * kLog2e;
-    const _Float16* kb = K + (b * seq + k0) * kD2;
-    u32x4v v[8];
-    loadPanelQ(kb, tid, v);
-    storePanelQ(ldsQ, tid, v);
+    for (int ks = 0; ks < KS; ++ks) xq[ks] = *reinterpret_cast<const f16x8*>(Q + qrow * D + ks * 16 + hl * 8);
+    for (int i = tid; i < keys; i += 256) lbias[i] = biasLog2(bias[k0 + i]);
+    const _Float16* kb = K + (b * seq + k0) * D;
+    u32x4v v[D / 16];
+    loadPanelQ<D>(kb, tid, v);
+    storePanelQ<D>(ldsQ, tid, v);
     __syncthreads();
     float m = -INFINITY, l = 0.0f;
     for (int p = 0; p < np; ++p) {
-        if (p + 1 < np) loadPanelQ(kb + static_cast<int64_t>(p + 1) * kPanelQ * kD2, tid, v);
-        const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ;
+        if (p + 1 < np) loadPanelQ<D>(kb + static_cast<int64_t>(p + 1) * kPanelQ * D, tid, v);
+        const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ<D>;
         f32x16 acc[4];
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
@@ -162,10 +186,10 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
             for (int r = 0; r < 16; ++r) acc[i][r] = 0.0f;
         }
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int i = 0; i < 4; ++i) {
-                const f16x8 a = *reinterpret_cast<const f16x8*>(pk + (i * 32 + l32) * kRowQ + ks * 16 + hl * 8);
+                const f16x8 a = *reinterpret_cast<const f16x8*>(pk + (i * 32 + l32) * kRowQ<D> + ks * 16 + hl * 8);
                 acc[i] = __builtin_amdgcn_mfma_f32_32x32x16_f16(a, xq[ks], acc[i], 0, 0, 0);
             }
         }
@@ -188,15 +212,18 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
         // are taken against a finite stand-in for the -inf max.
         const float mn = fmaxf(m, mb);
         const float ms = finiteOr0(mn);
-        float sb = 0.0f;
+        // Eight short sums: a quarter of one long one's rounding.
+        float sb[8];
 #pragma unroll
-        for (int i = 0; i < 4; ++i) {
+        for (int g = 0; g < 8; ++g) {
+            sb[g] = __builtin_amdgcn_exp2f(acc[g / 2][g % 2 * 8] - ms);
 #pragma unroll
-            for (int r = 0; r < 16; ++r) sb += __builtin_amdgcn_exp2f(acc[i][r] - ms);
+            for (int r = 1; r < 8; ++r) sb[g] += __builtin_amdgcn_exp2f(acc[g / 2][g % 2 * 8 + r] - ms);
         }
-        l = l * __builtin_amdgcn_exp2f(m - ms) + sb;
+        l = l * __builtin_amdgcn_exp2f(m - ms) +
+            (((sb[0] + sb[1]) + (sb[2] + sb[3])) + ((sb[4] + sb[5]) + (sb[6] + sb[7])));
         m = mn;
-        if (p + 1 < np) storePanelQ(ldsQ + ((p + 1) & 1) * kPanelHalvesQ, tid, v);
+        if (p + 1 < np) storePanelQ<D>(ldsQ + ((p + 1) & 1) * kPanelHalvesQ<D>, tid, v);
         __syncthreads();
     }
     const float mo = __shfl_xor(m, 32, 64);
@@ -207,67 +234,92 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
     return make_float2(mx, lt);
 }
 
-/// Row statistics of the 16 rows this lane's pass-2 accumulators hold,
-/// merged from NP key-range partials part[row * NP + i] (base 2), as one
-/// log-normalizer per row: rlm = max + log2(sum(exp2(v - max))), so pass 2
-/// writes exp2(v - rlm) = exp2(v - max) / sum with no multiply. A row whose
-/// scores are all -inf gets rlm = -inf (max -inf, sum 0): exp2(-inf - -inf)
-/// writes NaN, as the reference does.
-template <int NP>
-__device__ __forceinline__ void mergeStatsQ(const float2* __restrict__ part, int64_t r0, float (&rlm)[16]) {
+/// Row statistics of the 16 rows this lane's pass-2 accumulators hold: lane
+/// l32 merges row r0 + l32's nr partials pp (base 2; those past nr repeat the
+/// first) into shift and scale, which the lanes then pass around. Pass 2
+/// writes exp2(v - shift) * scale, scale 1 / sum(exp2(v - shift)). The shift is
+/// the row's max, or 0 for a row whose max is in [0, 64]: that subtraction has
+/// no rounding and is left out, and what then underflows, v < -126, is below
+/// float's normal range after the scale too.
+/// A log-normalizer max + log2(sum) in one float as the shift would save the
+/// multiply, and cost 2^-24 of its magnitude in every value of the row.
+/// A row whose scores are all -inf keeps max -inf: exp2(-inf - -inf) writes
+/// NaN, as the reference does. Returns whether every row's shift is 0.
+__device__ __forceinline__ bool mergeStatsQ(const float2 (&pp)[kMaxRangesQ], int nr, float (&shift)[16],
+                                            float (&scale)[16]) {
     const int hl = (threadIdx.x & 63) >> 5;
+    float m = pp[0].x;
+#pragma unroll
+    for (int i = 1; i < kMaxRangesQ; ++i) m = fmaxf(m, pp[i].x);
+    const bool plain = m >= 0.0f && m <= 64.0f;
+    const float sh = plain ? 0.0f : m;
+    const float ms = finiteOr0(sh);
+    float lt = 0.0f;
+#pragma unroll
+    for (int i = 0; i < kMaxRangesQ; ++i) lt += i < nr ? pp[i].y * __builtin_amdgcn_exp2f(pp[i].x - ms) : 0.0f;
+    const float sc = 1.0f / lt;
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        const float2* pr = part + (r0 + 8 * (r >> 2) + 4 * hl + (r & 3)) * NP;
-        float2 pp[NP];
-#pragma unroll
-        for (int i = 0; i < NP; ++i) pp[i] = pr[i];
-        float mx = pp[0].x;
-#pragma unroll
-        for (int i = 1; i < NP; ++i) mx = fmaxf(mx, pp[i].x);
-        const float ms = finiteOr0(mx);
-        float lt = 0.0f;
-#pragma unroll
-        for (int i = 0; i < NP; ++i) lt += pp[i].y * __builtin_amdgcn_exp2f(pp[i].x - ms);
-        rlm[r] = mx + __builtin_amdgcn_logf(lt);   // v_log_f32: log2
+        shift[r] = __shfl(sh, 8 * (r >> 2) + 4 * hl + (r & 3), 64);
+        scale[r] = __shfl(sc, 8 * (r >> 2) + 4 * hl + (r & 3), 64);
     }
+    return __all(plain);
 }
 
 /// Pass 2 over keys [k0, k0 + keys) of this wave's 32 rows r0..r0+31 of
-/// batch b: D = Q K^T per panel, written as exp2(v - max) / sum at once;
-/// each 32-lane half-wave stores one 128-byte line. RAGGED: Q, K and the
-/// bias are zero-padded copies of length seq of a sequence of length sseq;
-/// S is [batch][sseq][sseq] and only rows and keys below sseq are stored.
-template <bool RAGGED>
+/// batch b: D = Q K^T per panel, written as exp2(v - shift) * scale at once.
+/// RAGGED: Q, K and the bias are zero-padded copies of length seq of a sequence
+/// of length sseq; S is [batch][sseq][sseq] and only rows and keys below sseq
+/// are stored. QUADS (S 16-byte aligned, sseq a multiple of 4): MFMA column l
+/// of block j is key 4 l + j, so that a lane's four blocks hold four keys in a
+/// row and one store writes 512 bytes of each of two rows (8 x 1024 x 64: 15.1
+/// -> 13.9 us against 128 bytes); otherwise it is key 32 j + l and a store
+/// writes 128.
+/// Batches start at different panels: row blocks in step would write the same
+/// few columns of rows a power of two apart, which share memory channels (16 x
+/// 2048 x 128, both passes: 90.6 -> 77 us; x 64: 81 -> 67). Within a batch they
+/// stay in step, for K in the L2 (each row block apart: 84 and 74 us).
+template <int D, bool RAGGED, bool QUADS>
 __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                             const float* __restrict__ bias, float* __restrict__ S, int seq,
-                                            int sseq, float c2, int64_t b, int64_t r0, int k0, int keys,
-                                            const float (&rlm)[16], _Float16* ldsQ) {
+                                            int sseq, float c2, int64_t b, int rb, int64_t r0, int k0, int keys,
+                                            const float2* __restrict__ part, int nr, _Float16* ldsQ) {
     const int ld = RAGGED ? sseq : seq;           // S row length
     const int i0 = static_cast<int>(r0 - b * seq);   // first row within the batch
     const int tid = threadIdx.x;
     const int lane = tid & 63, l32 = lane & 31, hl = lane >> 5;
     const int np = keys / kPanelQ;
-    f16x8 aq[8];                                  // A operand: row r0 + l32
+    constexpr int KS = D / 16;
+    f16x8 aq[KS];                                 // A operand: row r0 + l32
 #pragma unroll
-    for (int ks = 0; ks < 8; ++ks) {
-        aq[ks] = *reinterpret_cast<const f16x8*>(Q + (r0 + l32) * kD2 + ks * 16 + hl * 8);
+    for (int ks = 0; ks < KS; ++ks) {
+        aq[ks] = *reinterpret_cast<const f16x8*>(Q + (r0 + l32) * D + ks * 16 + hl * 8);
     }
-    const _Float16* kb = K + (b * seq + k0) * kD2;
+    const _Float16* kb = K + (b * seq + k0) * D;
     // Stores: a scalar base per panel (row r0, key kc) plus a fixed lane
-    // offset per accumulator register r, the key sub-block j as an immediate.
+    // offset per accumulator register r.
+    const int lk = QUADS ? 4 * l32 : l32;         // this lane's key of block 0
+    constexpr int jk = QUADS ? 1 : 32;            // from block to block
     uint32_t soff[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
-        soff[r] = static_cast<uint32_t>(((8 * (r >> 2) + 4 * hl + (r & 3)) * ld + l32) * sizeof(float));
+        soff[r] = static_cast<uint32_t>(((8 * (r >> 2) + 4 * hl + (r & 3)) * ld + lk) * sizeof(float));
     }
-    u32x4v v[8];
-    loadPanelQ(kb, tid, v);
-    storePanelQ(ldsQ, tid, v);
+    float2 pp[kMaxRangesQ];
+#pragma unroll
+    for (int i = 0; i < kMaxRangesQ; ++i) pp[i] = part[(r0 + l32) * nr + (i < nr ? i : 0)];
+    u32x4v v[D / 16];
+    int at = static_cast<int>(b) % np;
+    loadPanelQ<D>(kb + static_cast<int64_t>(at) * kPanelQ * D, tid, v);
+    float shift[16], scale[16];
+    const bool plain = mergeStatsQ(pp, nr, shift, scale);
+    storePanelQ<D, QUADS>(ldsQ, tid, v);
     __syncthreads();
     for (int p = 0; p < np; ++p) {
-        if (p + 1 < np) loadPanelQ(kb + static_cast<int64_t>(p + 1) * kPanelQ * kD2, tid, v);
-        const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ;
+        const int kc = k0 + at * kPanelQ;
+        if (++at == np) at = 0;
+        if (p + 1 < np) loadPanelQ<D>(kb + static_cast<int64_t>(at) * kPanelQ * D, tid, v);
+        const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ<D>;
         f32x16 acc[4];
 #pragma unroll
         for (int j = 0; j < 4; ++j) {
@@ -275,102 +327,160 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
             for (int r = 0; r < 16; ++r) acc[j][r] = 0.0f;
         }
 #pragma unroll
-        for (int ks = 0; ks < 8; ++ks) {
+        for (int ks = 0; ks < KS; ++ks) {
 #pragma unroll
             for (int j = 0; j < 4; ++j) {
-                const f16x8 x = *reinterpret_cast<const f16x8*>(pk + (j * 32 + l32) * kRowQ + ks * 16 + hl * 8);
+                const f16x8 x = *reinterpret_cast<const f16x8*>(pk + (j * 32 + l32) * kRowQ<D> + ks * 16 + hl * 8);
                 acc[j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(aq[ks], x, acc[j], 0, 0, 0);
             }
         }
-        const int kc = k0 + p * kPanelQ;
         float bj[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bj[j] = bias[kc + j * 32 + l32] * kLog2e;
+        for (int j = 0; j < 4; ++j) bj[j] = biasLog2(bias[kc + lk + j * jk]);
         char* sb = reinterpret_cast<char*>(S + (b * ld + i0) * static_cast<int64_t>(ld) + kc);
+        auto store = [&](auto value) {
 #pragma unroll
-        for (int r = 0; r < 16; ++r) {
+            for (int r = 0; r < 16; ++r) {
+                if (RAGGED && i0 + 8 * (r >> 2) + 4 * hl + (r & 3) >= sseq) continue;
+                f32x4 out;
 #pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                if (RAGGED && (i0 + 8 * (r >> 2) + 4 * hl + (r & 3) >= sseq || kc + j * 32 + l32 >= sseq)) continue;
-                *reinterpret_cast<float*>(sb + soff[r] + j * 32 * sizeof(float)) =
-                    __builtin_amdgcn_exp2f(__builtin_fmaf(acc[j][r], c2, bj[j]) - rlm[r]);
+                for (int j = 0; j < 4; ++j) out[j] = value(__builtin_fmaf(acc[j][r], c2, bj[j]), r);
+                if (QUADS) {
+                    if (!RAGGED || kc + lk < sseq) *reinterpret_cast<f32x4*>(sb + soff[r]) = out;
+                } else {
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        if (kc + lk + j * jk < sseq) *reinterpret_cast<float*>(sb + soff[r] + j * jk * sizeof(float)) = out[j];
+                    }
+                }
             }
+        };
+        if (plain) {
+            store([&](float v, int r) { return __builtin_amdgcn_exp2f(v) * scale[r]; });
+        } else {
+            store([&](float v, int r) { return __builtin_amdgcn_exp2f(v - shift[r]) * scale[r]; });
         }
-        if (p + 1 < np) storePanelQ(ldsQ + ((p + 1) & 1) * kPanelHalvesQ, tid, v);
+        if (p + 1 < np) storePanelQ<D, QUADS>(ldsQ + ((p + 1) & 1) * kPanelHalvesQ<D>, tid, v);
         __syncthreads();
     }
 }
 
+template <int D>
 __global__ __launch_bounds__(256, 2) void scoreStatsQ(const _Float16* __restrict__ Q,
                                                       const _Float16* __restrict__ K,
                                                       const float* __restrict__ bias,
-                                                      float2* __restrict__ part, int seq, float c2) {
+                                                      float2* __restrict__ part, int seq, int nr, int per, float c2) {
     extern __shared__ __align__(16) _Float16 ldsQ[];
     int64_t b;
-    int rb, kh;
-    blockOfQ(seq / 128, b, rb, kh);
+    int rb, kr, k0, keys;
+    blockOfQ(seq, nr, per, b, rb, kr, k0, keys);
     int64_t qrow;
-    const float2 st = statsRangeQ(Q, K, bias, seq, c2, b, rb, kh * (seq / 2), seq / 2, ldsQ, qrow);
-    if (((threadIdx.x & 63) >> 5) == 0) part[qrow * 2 + kh] = st;
+    const float2 st = statsRangeQ<D>(Q, K, bias, seq, c2, b, rb, k0, keys, ldsQ, qrow);
+    if (((threadIdx.x & 63) >> 5) == 0) part[qrow * nr + kr] = st;
 }
 
-template <bool RAGGED>
+template <int D, bool RAGGED, bool QUADS>
 __global__ __launch_bounds__(256, 2) void scoreStoreQ(const _Float16* __restrict__ Q,
                                                       const _Float16* __restrict__ K,
                                                       const float* __restrict__ bias,
                                                       const float2* __restrict__ part, float* __restrict__ S,
-                                                      int seq, int sseq, float c2) {
+                                                      int seq, int sseq, int nr, int per,
+                                                      float c2) {
     extern __shared__ __align__(16) _Float16 ldsQ[];
     int64_t b;
-    int rb, kh;
-    blockOfQ(seq / 128, b, rb, kh);
+    int rb, kr, k0, keys;
+    blockOfQ(seq, nr, per, b, rb, kr, k0, keys);
     const int wave = __builtin_amdgcn_readfirstlane(static_cast<int>(threadIdx.x >> 6));
     const int64_t r0 = b * seq + static_cast<int64_t>(rb) * 128 + wave * 32;   // wave-uniform
-    float rlm[16];
-    mergeStatsQ<2>(part, r0, rlm);
-    storeRangeQ<RAGGED>(Q, K, bias, S, seq, sseq, c2, b, r0, kh * (seq / 2), seq / 2, rlm, ldsQ);
+    storeRangeQ<D, RAGGED, QUADS>(Q, K, bias, S, seq, sseq, c2, b, rb, r0, k0, keys, part, nr, ldsQ);
 }
 
-/// Both passes over p's (padded) Q, K and bias; `ragged` > 0 stores only
-/// rows and keys below it into p->s laid out [batch][ragged][ragged].
-int launchQ(const mlkd_score_softmax* p, hipStream_t st, int64_t ragged = 0) {
-    const size_t ldsStats = kLdsStoreQ + static_cast<size_t>(p->seq / 2) * sizeof(float);
+/// Panels of each key range but the last: those that take the fewest panel
+/// times, a workgroup's start (Q, its first panel, the statistics) counted as
+/// two, over the 512 workgroups the chip holds at once (two ranges against up
+/// to eight: 1 x 2048 x 128 36.7 -> 15.4 us, 1 x 1024 x 128 20.8 -> 9.7, 8 x
+/// 1024 x 64 19.6 -> 14.4, 4 x 512 x 64 11.0 -> 7.8). `most` is the number of
+/// ranges there is room for. Shapes with a choice of launch forms keep to form
+/// 0's two ranges below 8 panels.
+int panelsPerRange(const mlkd_score_softmax* p, int most) {
+    const int64_t panels = p->seq / kPanelQ, rows = p->batch * panels;
+    if (p->dim == 128 && p->seq % 256 == 0 && panels < 8) return static_cast<int>(panels / 2);
+    int64_t best = 0, per = panels;
+    for (int64_t nr = 1; nr <= std::min<int64_t>(most, panels); ++nr) {
+        const int64_t each = (panels + nr - 1) / nr;
+        const int64_t slots = each <= 24 ? 512 : 256;   // past 24 panels a bias in LDS leaves room for one a CU
+        const int64_t t = (rows * ((panels + each - 1) / each) + slots - 1) / slots * (each + 2);
+        if (nr > 1 && t >= best) continue;
+        best = t;
+        per = each;
+    }
+    return static_cast<int>(per);
+}
+
+int rangesQ(const mlkd_score_softmax* p, int most = kMaxRangesQ) {
+    const int64_t per = panelsPerRange(p, most);
+    return static_cast<int>((p->seq / kPanelQ + per - 1) / per);
+}
+
+/// Both passes over p's (padded) Q, K and bias, at most `most` key ranges per
+/// row block with their partials in p->scratch; `ragged` > 0 stores only rows and keys
+/// below it into p->s laid out [batch][ragged][ragged].
+template <int D>
+int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragged) {
     // Once per process; a function-local static initializes thread-safely.
     static const bool attrs = [] {
-        const size_t maxStats = kLdsStoreQ + static_cast<size_t>(kMaxSeqQ / 2) * sizeof(float);
-        return hipFuncSetAttribute(reinterpret_cast<const void*>(scoreStatsQ), hipFuncAttributeMaxDynamicSharedMemorySize,
-                                   static_cast<int>(maxStats)) == hipSuccess &&
-               hipFuncSetAttribute(reinterpret_cast<const void*>(scoreStoreQ<false>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsStoreQ)) == hipSuccess &&
-               hipFuncSetAttribute(reinterpret_cast<const void*>(scoreStoreQ<true>),
-                                   hipFuncAttributeMaxDynamicSharedMemorySize, static_cast<int>(kLdsStoreQ)) == hipSuccess;
+        const int maxStats = static_cast<int>(kLdsStoreQ<D> + static_cast<size_t>(kMaxSeqQ) * sizeof(float));
+        for (const void* fn : {reinterpret_cast<const void*>(scoreStatsQ<D>),
+                               reinterpret_cast<const void*>(scoreStoreQ<D, false, true>),
+                               reinterpret_cast<const void*>(scoreStoreQ<D, true, true>),
+                               reinterpret_cast<const void*>(scoreStoreQ<D, true, false>)}) {
+            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxStats) != hipSuccess) return false;
+        }
+        return true;
     }();
     if (!attrs) return MLKD_RT_LAUNCH;
-    const unsigned blocks = static_cast<unsigned>(p->batch * (p->seq / 128) * 2);
+    const int per = panelsPerRange(p, most) * kPanelQ;
+    const size_t ldsStats = kLdsStoreQ<D> + static_cast<size_t>(per) * sizeof(float);
+    const int nr = rangesQ(p, most);
+    const dim3 grid(static_cast<unsigned>(p->batch * (p->seq / kPanelQ) * nr));
     // Both passes work in base 2: v2 = acc * (log2(e) / div) + bias * log2(e),
     // exp(v - max) = exp2(v2 - max2).
     const float c2 = static_cast<float>(1.4426950408889634 / p->div);
-    hipLaunchKernelGGL(scoreStatsQ, dim3(blocks), dim3(256), ldsStats, st, static_cast<const _Float16*>(p->q),
+    hipLaunchKernelGGL(scoreStatsQ<D>, grid, dim3(256), ldsStats, st, static_cast<const _Float16*>(p->q),
                        static_cast<const _Float16*>(p->k), static_cast<const float*>(p->bias),
-                       static_cast<float2*>(p->scratch), static_cast<int>(p->seq), c2);
-    hipLaunchKernelGGL(ragged > 0 ? scoreStoreQ<true> : scoreStoreQ<false>, dim3(blocks), dim3(256), kLdsStoreQ, st,
+                       static_cast<float2*>(p->scratch), static_cast<int>(p->seq), nr, per, c2);
+    const int64_t sseq = ragged > 0 ? ragged : p->seq;
+    auto store = scoreStoreQ<D, true, false>;
+    if (sseq % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s) & 15u) == 0) {
+        store = ragged > 0 ? scoreStoreQ<D, true, true> : scoreStoreQ<D, false, true>;
+    }
+    hipLaunchKernelGGL(store, grid, dim3(256), kLdsStoreQ<D>, st,
                        static_cast<const _Float16*>(p->q), static_cast<const _Float16*>(p->k),
                        static_cast<const float*>(p->bias), static_cast<const float2*>(p->scratch),
                        static_cast<float*>(p->s), static_cast<int>(p->seq),
-                       static_cast<int>(ragged > 0 ? ragged : p->seq), c2);
+                       static_cast<int>(sseq), nr, per, c2);
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
 }
 
+/// `div` is held to where 1 / div times log2(e) is a normal float.
+/// Head dim 64 takes it from 512 keys, and more rows than that: with fewer it
+/// gains nothing (3 x 256: 7.9 against 7.4 us, 1 x 512: 8.0 and 7.7, 2 x 512:
+/// 7.8 and 8.3) and with fewer keys its error is the larger (16 x 128: 1.30e-7
+/// against 1.24e-7; 2 x 512: 1.38e-7 and 1.40e-7, 8 x 1024: 1.42e-7 and 1.44e-7).
 bool twoPassApplies(const mlkd_score_softmax* p) {
+    const double size = p->div < 0 ? -p->div : p->div;
+    if (!(size >= 1e-30 && size <= 1e30)) return false;
     return p->qk_dtype == MLKD_F16 && p->bias_dtype == MLKD_F32 && p->s_dtype == MLKD_F32 &&
-           p->dim == kD2 && p->seq % 256 == 0 && p->seq > 0 && p->seq <= kMaxSeqQ &&
+           (p->dim == 64 || p->dim == 128) && p->seq % kPanelQ == 0 && p->seq > 0 && p->seq <= kMaxSeqQ &&
+           (p->dim == 128 || (p->seq >= 512 && p->batch * p->seq > 512)) &&
            (reinterpret_cast<uintptr_t>(p->q) & 15u) == 0 && (reinterpret_cast<uintptr_t>(p->k) & 15u) == 0 &&
-           p->batch * (p->seq / 128) * 2 <= 0x7FFFFFFF;
+           p->batch * (p->seq / kPanelQ) * 8 <= 0x7FFFFFFF;
 }
 
-/// Row statistics partials: one (max, sum) pair per row and key half.
-int64_t scratch2(const mlkd_score_softmax* p) {
-    return p->batch * p->seq * 2 * static_cast<int64_t>(sizeof(float2));
+/// Row statistics partials of nr key ranges: one (max, sum) pair per row and
+/// range.
+int64_t statsBytes(const mlkd_score_softmax* p, int nr) {
+    return p->batch * p->seq * nr * static_cast<int64_t>(sizeof(float2));
 }
 
 template <typename T>
@@ -425,42 +535,74 @@ __global__ __launch_bounds__(256) void padBias(const float* __restrict__ src, in
     }
 }
 
-/// The padded two-pass launch: sequence length rounded up to 256 (at most
-/// kMaxSeqQ), for shapes the two passes would take but for the length.
-/// Q, K and the bias are copied into the workspace (q.s stays the caller's
-/// S: pass 2 stores only its rows and keys). It is faster than the general
-/// kernels at every size measured, down to 1x100x128 (general: 41 us).
-bool padScore(const mlkd_score_softmax* p, mlkd_score_softmax& q) {
-    if (p->work == nullptr || p->seq % 256 == 0) return false;
-    q = *p;
-    q.seq = (p->seq + 255) / 256 * 256;
-    if (q.seq > kMaxSeqQ) return false;
-    unsigned char* w = static_cast<unsigned char*>(p->work);
-    const size_t qk = static_cast<size_t>(p->batch * q.seq * kD2) * sizeof(_Float16);
-    q.q = w;
-    q.k = w + qk;
-    q.bias = w + 2 * qk;
-    q.scratch = w + 2 * qk + static_cast<size_t>(q.seq) * sizeof(float);
-    q.scratch_bytes = scratch2(&q);
-    q.work = nullptr;
-    q.work_bytes = 0;
-    const int64_t need = static_cast<int64_t>(2 * qk + static_cast<size_t>(q.seq) * sizeof(float)) + q.scratch_bytes;
-    return twoPassApplies(&q) && p->work_bytes >= need && (reinterpret_cast<uintptr_t>(p->q) & 15u) == 0 &&
-           (reinterpret_cast<uintptr_t>(p->k) & 15u) == 0;
+/// Workspace bytes of the two passes: nothing but the partials where p's
+/// sequence is whole panels, otherwise copies of Q, K and the bias padded to a
+/// whole number first. 0 where the two passes don't run on a workspace.
+/// `q`, if given, is set up to run in the workspace p->work.
+int64_t workBytes(const mlkd_score_softmax* p, mlkd_score_softmax* q = nullptr) {
+    mlkd_score_softmax w = *p;
+    w.seq = (p->seq + kPanelQ - 1) / kPanelQ * kPanelQ;
+    if (!twoPassApplies(&w)) return 0;
+    int64_t at = 0;
+    unsigned char* base = static_cast<unsigned char*>(p->work);
+    if (w.seq != p->seq) {
+        // Off the panels at dim 64 the general kernels run.
+        if (p->dim != 128) return 0;
+        const int64_t qk = p->batch * w.seq * p->dim * static_cast<int64_t>(sizeof(_Float16));
+        w.q = base;
+        w.k = base + qk;
+        w.bias = base + 2 * qk;
+        at = 2 * qk + w.seq * static_cast<int64_t>(sizeof(float));
+    }
+    w.scratch = base + at;
+    w.scratch_bytes = statsBytes(&w, rangesQ(&w));
+    if (q != nullptr) *q = w;
+    return at + w.scratch_bytes;
 }
 
-int launchPaddedQ(const mlkd_score_softmax* p, const mlkd_score_softmax& q, hipStream_t st) {
-    const int64_t pieces = p->batch * q.seq * 16;
-    const unsigned g = static_cast<unsigned>(std::min<int64_t>((pieces + 255) / 256, 16384));
-    hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->q), p->batch, p->seq,
-                       static_cast<u32x4v*>(const_cast<void*>(q.q)), q.seq);
-    hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->k), p->batch, p->seq,
-                       static_cast<u32x4v*>(const_cast<void*>(q.k)), q.seq);
-    hipLaunchKernelGGL(padBias, dim3(static_cast<unsigned>((q.seq + 255) / 256)), dim3(256), 0, st,
-                       static_cast<const float*>(p->bias), p->seq, static_cast<float*>(const_cast<void*>(q.bias)),
-                       q.seq);
-    if (hipGetLastError() != hipSuccess) return MLKD_RT_LAUNCH;
-    return launchQ(&q, st, p->seq);
+/// Scratch a run of the two passes is always given: dim 128, whole pairs of
+/// panels, two key ranges. Elsewhere, and for more ranges, they take a
+/// workspace where there is one.
+int64_t requiredBytes(const mlkd_score_softmax* p) {
+    return p->dim == 128 && p->seq % (2 * kPanelQ) == 0 && twoPassApplies(p) ? statsBytes(p, 2) : 0;
+}
+
+/// Whether p runs in two passes, with q and the most key ranges set up.
+bool runsTwoPass(const mlkd_score_softmax* p, int variant, mlkd_score_softmax& q, int& most) {
+    if (variant == 1) return false;
+    const int64_t work = workBytes(p, &q);
+    if (work > 0 && p->work != nullptr && (reinterpret_cast<uintptr_t>(p->work) & 15u) == 0 && p->work_bytes >= work) {
+        most = kMaxRangesQ;
+        return true;
+    }
+    const int64_t need = requiredBytes(p);
+    if (need > 0 && p->scratch != nullptr && (reinterpret_cast<uintptr_t>(p->scratch) & 7u) == 0 &&
+        p->scratch_bytes >= need) {
+        q = *p;
+        most = 2;
+        return true;
+    }
+    return false;
+}
+
+int launchTwoPass(const mlkd_score_softmax* p, const mlkd_score_softmax& q, int most, hipStream_t st) {
+    const int64_t ragged = q.seq == p->seq ? 0 : p->seq;
+    if (ragged > 0) {
+        // Copies padded with zero rows and -inf bias, and both passes over
+        // them, are faster than the general kernels at every size measured,
+        // down to 1 x 100 x 128 (general: 41 us).
+        const int64_t pieces = p->batch * q.seq * 16;
+        const unsigned g = static_cast<unsigned>(std::min<int64_t>((pieces + 255) / 256, 16384));
+        hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->q), p->batch, p->seq,
+                           static_cast<u32x4v*>(const_cast<void*>(q.q)), q.seq);
+        hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->k), p->batch, p->seq,
+                           static_cast<u32x4v*>(const_cast<void*>(q.k)), q.seq);
+        hipLaunchKernelGGL(padBias, dim3(static_cast<unsigned>((q.seq + 255) / 256)), dim3(256), 0, st,
+                           static_cast<const float*>(p->bias), p->seq, static_cast<float*>(const_cast<void*>(q.bias)),
+                           q.seq);
+        if (hipGetLastError() != hipSuccess) return MLKD_RT_LAUNCH;
+    }
+    return p->dim == 64 ? launchQ<64>(&q, most, st, ragged) : launchQ<128>(&q, most, st, ragged);
 }
 
 // 0: the best form for the shape (the two-pass query-stationary form where
@@ -471,29 +613,23 @@ int gScoreVariant = 0;
 
 extern "C" void mlkd_score_set_variant(int variant) { gScoreVariant = variant; }
 
-extern "C" int64_t mlkd_score_scratch_bytes(const mlkd_score_softmax* p) {
-    return p != nullptr && twoPassApplies(p) ? scratch2(p) : 0;
+extern "C" int mlkd_score_ranges(const mlkd_score_softmax* p) {
+    mlkd_score_softmax q;
+    return workBytes(p, &q) > 0 ? rangesQ(&q) : 0;
 }
 
+extern "C" int64_t mlkd_score_scratch_bytes(const mlkd_score_softmax* p) { return p != nullptr ? requiredBytes(p) : 0; }
+
 extern "C" int64_t mlkd_score_pad_bytes(const mlkd_score_softmax* p) {
-    if (p == nullptr) return 0;
-    mlkd_score_softmax probe = *p;
-    probe.work = reinterpret_cast<void*>(uintptr_t{1} << 12);
-    probe.work_bytes = INT64_MAX;
-    mlkd_score_softmax q;
-    if (!padScore(&probe, q)) return 0;
-    const int64_t qk = p->batch * q.seq * kD2 * static_cast<int64_t>(sizeof(_Float16));
-    return 2 * qk + q.seq * static_cast<int64_t>(sizeof(float)) + scratch2(&q);
+    const int64_t work = p != nullptr ? workBytes(p) : 0;
+    return work > (p != nullptr ? requiredBytes(p) : 0) ? work : 0;
 }
 
 extern "C" const char* mlkd_score_kernel_names(const mlkd_score_softmax* p) {
     static thread_local char name[160];
-    const int variant = p->variant >= 0 ? p->variant : gScoreVariant;
-    if (mlkd_score_softmax q; variant != 1 && padScore(p, q)) return "scoreStatsQ+scoreStoreQ";
-    if (variant != 1 && twoPassApplies(p) && p->scratch != nullptr &&
-        (reinterpret_cast<uintptr_t>(p->scratch) & 7u) == 0 && p->scratch_bytes >= scratch2(p)) {
-        return "scoreStatsQ+scoreStoreQ";
-    }
+    mlkd_score_softmax q;
+    int most;
+    if (runsTwoPass(p, p->variant >= 0 ? p->variant : gScoreVariant, q, most)) return "scoreStatsQ+scoreStoreQ";
     const bool fast = p->qk_dtype == MLKD_F16 && p->bias_dtype == MLKD_F32 && p->s_dtype == MLKD_F32 &&
                       p->seq % 128 == 0 && p->dim % 16 == 0 && p->dim > 0 && p->seq < (1 << 20) &&
                       (reinterpret_cast<uintptr_t>(p->q) & 15u) == 0 &&
@@ -518,11 +654,9 @@ extern "C" int mlkd_launch_score_softmax(const mlkd_score_softmax* p, void* stre
     if (p->batch == 0 || p->seq == 0) return 0;
     hipStream_t st = static_cast<hipStream_t>(stream);
     const int variant = p->variant >= 0 ? p->variant : gScoreVariant;
-    if (variant != 1 && twoPassApplies(p) && p->scratch != nullptr &&
-        (reinterpret_cast<uintptr_t>(p->scratch) & 7u) == 0 && p->scratch_bytes >= scratch2(p)) {
-        return launchQ(p, st);
-    }
-    if (mlkd_score_softmax q; variant != 1 && padScore(p, q)) return launchPaddedQ(p, q, st);
+    mlkd_score_softmax q;
+    int most;
+    if (runsTwoPass(p, variant, q, most)) return launchTwoPass(p, q, most, st);
     const bool fast = p->qk_dtype == MLKD_F16 && p->bias_dtype == MLKD_F32 && p->s_dtype == MLKD_F32 &&
                       p->seq % 128 == 0 && p->dim % 16 == 0 && p->dim > 0 && p->seq < (1 << 20) &&
                       (reinterpret_cast<uintptr_t>(p->q) & 15u) == 0 &&

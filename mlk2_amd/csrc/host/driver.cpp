@@ -275,6 +275,26 @@ namespace {
 size_t align256(size_t v) { return (v + 255) & ~static_cast<size_t>(255); }
 }  // namespace
 
+int64_t HipLoadedKernel::stepScratch(RunScratch& rs, size_t si, int64_t need, int64_t want, void* stream,
+                                     void** ptr) const {
+    std::lock_guard<std::mutex> g(scratchLock_);
+    void*& p = rs.step[si];
+    int64_t& bytes = rs.stepBytes[si];
+    if (bytes < (need > 0 ? need : want)) {
+        if (p != nullptr) mlkd_rt_free(p);
+        bytes = 0;
+        if (want > need && mlkd_rt_malloc_spare(&p, static_cast<size_t>(want), stream) == 0) {
+            bytes = want;
+        } else if (need > 0 && mlkd_rt_malloc(&p, static_cast<size_t>(need)) == 0) {
+            bytes = need;
+        } else {
+            p = nullptr;
+        }
+    }
+    *ptr = p;
+    return bytes;
+}
+
 void HipLoadedKernel::fillScoreParams(const Step& st, const std::vector<void*>& ptr, mlkd_score_softmax& p) const {
     p.variant = st.variant;
     p.q = ptr[st.q];
@@ -438,10 +458,10 @@ int HipLoadedKernel::arenaLayout(const DeviceBinding* binds, int64_t elements, c
               std::to_string(arena.bytes);
         return MLKHIP_REFUSED;
     }
-    // Workspaces a step can do without (GEMM shapes off the MFMA tiles,
-    // score-softmax lengths off the two-pass blocks) take the room that is
-    // left, in step order; a step whose workspace does not fit runs on the
-    // general kernels.
+    // Workspaces a step can do without (aligned copies of a GEMM's operands
+    // or the sums of its K ranges, score-softmax statistics and padded copies)
+    // take the room that is left, in step order; a step whose workspace does
+    // not fit runs on the kernels that need none.
     padOff.assign(plan_.steps.size(), SIZE_MAX);
     for (size_t si = 0; si < plan_.steps.size(); ++si) {
         const Step& st = plan_.steps[si];
@@ -607,17 +627,8 @@ int HipLoadedKernel::runDevice(const DeviceBinding* binds, int n, const double* 
                     p.work = arena->base + padOff[si];
                     p.work_bytes = need;
                 } else if (need > 0 && arena == nullptr) {
-                    std::lock_guard<std::mutex> g(scratchLock_);
-                    if (rs->step[si] == nullptr || rs->stepBytes[si] < need) {
-                        if (rs->step[si] != nullptr) mlkd_rt_free(rs->step[si]);
-                        rs->step[si] = nullptr;
-                        rs->stepBytes[si] = 0;
-                        if (mlkd_rt_malloc(&rs->step[si], static_cast<size_t>(need)) != 0) rs->step[si] = nullptr;
-                        else rs->stepBytes[si] = need;
-                    }
                     // Without the workspace the general kernel runs the step.
-                    p.work = rs->step[si];
-                    p.work_bytes = rs->stepBytes[si];
+                    p.work_bytes = stepScratch(*rs, si, 0, need, stream, &p.work);
                 }
                 rc = mlkd_launch_gemm(&p, stream);
                 break;
@@ -677,42 +688,25 @@ int HipLoadedKernel::runDevice(const DeviceBinding* binds, int n, const double* 
                 }
                 mlkd_score_softmax p;
                 fillScoreParams(st, ptr, p);
-                if (const int64_t need = mlkd_score_scratch_bytes(&p); need > 0 && arena != nullptr) {
-                    p.scratch = arena->base + stepOff[si];
-                    p.scratch_bytes = need;
-                } else if (need > 0) {
-                    std::lock_guard<std::mutex> g(scratchLock_);
-                    if (rs->step[si] == nullptr || rs->stepBytes[si] < need) {
-                        if (rs->step[si] != nullptr) mlkd_rt_free(rs->step[si]);
-                        rs->step[si] = nullptr;
-                        if (mlkd_rt_malloc(&rs->step[si], static_cast<size_t>(need)) != 0) {
-                            rs->step[si] = nullptr;
-                            why = "score-softmax scratch allocation failed";
-                            return MLKHIP_RUNTIME;
-                        }
-                        rs->stepBytes[si] = need;
+                // `need` is scratch the step can't run without; with a workspace
+                // of `pad` bytes it runs faster (both may be one allocation).
+                const int64_t need = mlkd_score_scratch_bytes(&p), pad = mlkd_score_pad_bytes(&p);
+                if (arena != nullptr) {
+                    if (need > 0) {
+                        p.scratch = arena->base + stepOff[si];
+                        p.scratch_bytes = need;
                     }
-                    p.scratch = rs->step[si];
-                    p.scratch_bytes = rs->stepBytes[si];
-                } else if (const int64_t pad = mlkd_score_pad_bytes(&p); pad > 0 && arena != nullptr) {
                     if (padOff[si] != SIZE_MAX) {
                         p.work = arena->base + padOff[si];
                         p.work_bytes = pad;
                     }
-                } else if (pad > 0) {
-                    // A sequence length off the two-pass blocks runs on
-                    // zero-padded copies, as for GEMM shapes off the MFMA
-                    // tiles; without the workspace the general kernels run.
-                    std::lock_guard<std::mutex> g(scratchLock_);
-                    if (rs->step[si] == nullptr || rs->stepBytes[si] < pad) {
-                        if (rs->step[si] != nullptr) mlkd_rt_free(rs->step[si]);
-                        rs->step[si] = nullptr;
-                        rs->stepBytes[si] = 0;
-                        if (mlkd_rt_malloc(&rs->step[si], static_cast<size_t>(pad)) != 0) rs->step[si] = nullptr;
-                        else rs->stepBytes[si] = pad;
+                } else if (need > 0 || pad > 0) {
+                    p.work_bytes = p.scratch_bytes = stepScratch(*rs, si, need, pad, stream, &p.work);
+                    p.scratch = p.work;
+                    if (p.work_bytes < need) {
+                        why = "score-softmax scratch allocation failed";
+                        return MLKHIP_RUNTIME;
                     }
-                    p.work = rs->step[si];
-                    p.work_bytes = rs->stepBytes[si];
                 }
                 rc = mlkd_launch_score_softmax(&p, stream);
                 break;

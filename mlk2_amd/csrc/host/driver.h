@@ -117,6 +117,10 @@ private:
     };
     RunScratch& scratchFor(void* stream) const;  // caller holds scratchLock_
     static void freeScratch(RunScratch& rs);
+    /// Bytes of rs.step[si] (at *ptr), allocated on first use: `want` where the step can
+    /// do without it and they can be had (not while `stream` is captured),
+    /// otherwise `need`; less than that when the allocation fails.
+    int64_t stepScratch(RunScratch& rs, size_t si, int64_t need, int64_t want, void* stream, void** ptr) const;
     /// Offsets of a run's scratch in `arena`; refuses what does not fit or
     /// needs a host read-back.
     int arenaLayout(const DeviceBinding* binds, int64_t elements, const ScratchArena& arena,

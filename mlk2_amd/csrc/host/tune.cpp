@@ -402,20 +402,31 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
             break;
         }
         case StepKind::ScoreSoftmax: {
-            // Output scores; the two-pass form (dim 128, seq % 256 == 0)
-            // gives each workgroup of a pass 128 rows x half the keys. A
-            // sequence off the 256-row blocks runs it on copies padded to
-            // seq' (a multiple of 256).
+            // Output scores; the two-pass form gives each workgroup of a pass
+            // 128 rows x one of the key ranges, over a sequence rounded up to
+            // whole 128-key panels.
+            auto code = [&](uint32_t b) {
+                const Dtype d = km.buffers[b].dtype;
+                return d == Dtype::F32 ? MLKD_F32 : d == Dtype::F16 ? MLKD_F16 : MLKD_F64;
+            };
             instances = st.batch * st.seq * st.seq;
-            const int64_t sp = (st.seq + 255) / 256 * 256;
-            const bool padded = st.seq % 256 != 0;
-            const bool twoPass = st.dim == 128 && sp <= 8192 && st.variant != 1;
-            workgroups = twoPass ? st.batch * (sp / 128) * 2 : st.batch * ((st.seq + 63) / 64) * ((st.seq + 127) / 128);
-            perGroup = twoPass ? 64 * sp : 64 * 128;
+            mlkd_score_softmax p{};
+            p.qk_dtype = code(st.q);
+            p.bias_dtype = code(st.bias);
+            p.s_dtype = code(st.s);
+            p.batch = st.batch;
+            p.seq = st.seq;
+            p.dim = st.dim;
+            p.div = st.div;
+            const int64_t sp = (st.seq + 127) / 128 * 128;
+            const int ranges = st.variant != 1 ? mlkd_score_ranges(&p) : 0;
+            workgroups = ranges > 0 ? st.batch * (sp / 128) * ranges
+                                    : st.batch * ((st.seq + 63) / 64) * ((st.seq + 127) / 128);
+            perGroup = ranges > 0 ? (128 * sp + ranges - 1) / ranges : 64 * 128;
             covered = workgroups * perGroup >= instances;
-            form = !twoPass ? "64 x 128 score tiles, then row softmax"
-                   : padded ? "128-row blocks x key halves, per pass, over zero-padded Q and K"
-                            : "128-row blocks x key halves, per pass";
+            form = ranges == 0     ? "64 x 128 score tiles, then row softmax"
+                   : sp != st.seq  ? "128-row blocks x key ranges, per pass, over zero-padded Q and K"
+                                   : "128-row blocks x key ranges, per pass";
             break;
         }
         case StepKind::Fail:
