@@ -108,8 +108,8 @@ const char* mlkd_softmax_kernel_name(const mlkd_softmax* p);
 const char* mlkd_score_kernel_names(const mlkd_score_softmax* p);
 /// Workspace bytes (16-byte aligned) that let mlkd_launch_score_softmax take
 /// the two-pass form where it is not given scratch for it (head dim 64,
-/// sequences off whole pairs of 128-key panels, those off the panels on
-/// zero-padded copies), or split the keys further; 0 when none applies.
+/// sequences off whole pairs of 128-key panels), or split the keys further; 0
+/// when none applies.
 int64_t mlkd_score_pad_bytes(const mlkd_score_softmax* p);
 /// Process default of the f16 GEMM launch form (8: direct-to-LDS ring with 8
 /// waves of 16x16x32 tiles, the default; 7: the same ring with 4 waves of

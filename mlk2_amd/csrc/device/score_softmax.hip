@@ -114,12 +114,19 @@ __device__ __forceinline__ float biasLog2(float b) {
     return __builtin_isinf(t) && !__builtin_isinf(b) ? __builtin_copysignf(3.402823466e+38f, t) : t;
 }
 
-/// 256 threads: global -> registers for one 128-key panel (D / 16 16-byte
-/// pieces each), which is contiguous in K.
-template <int D>
-__device__ __forceinline__ void loadPanelQ(const _Float16* __restrict__ k, int tid, u32x4v (&v)[D / 16]) {
+/// 256 threads: global -> registers for the 128-key panel of K (its batch's
+/// first row) at row `at`, D / 16 16-byte pieces each, contiguous in K. RAGGED:
+/// rows from `rows` on repeat the last one.
+template <int D, bool RAGGED>
+__device__ __forceinline__ void loadPanelQ(const _Float16* __restrict__ k, int at, int rows, int tid,
+                                           u32x4v (&v)[D / 16]) {
+    const _Float16* kb = k + static_cast<int64_t>(at) * D;
 #pragma unroll
-    for (int j = 0; j < D / 16; ++j) v[j] = *reinterpret_cast<const u32x4v*>(k + (j * 256 + tid) * 8);
+    for (int j = 0; j < D / 16; ++j) {
+        const int c = j * 256 + tid;
+        const int piece = RAGGED ? min(c / (D / 8), rows - 1 - at) * (D / 8) + c % (D / 8) : c;
+        v[j] = *reinterpret_cast<const u32x4v*>(kb + piece * 8);
+    }
 }
 
 /// Registers -> LDS: key i of the panel to row i, or (QUADS) to row
@@ -156,9 +163,9 @@ __device__ __forceinline__ void blockOfQ(int seq, int nr, int per, int64_t& b, i
 /// running max and sum(exp2(v - max)) of its query; the lane 32 away holds
 /// the other keys of the same query and the pair is combined at the end.
 /// Returns (max, sum) of query row `qrow` in base 2 (both half-waves agree).
-template <int D>
+template <int D, bool RAGGED>
 __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
-                                              const float* __restrict__ bias, int seq, float c2, int64_t b,
+                                              const float* __restrict__ bias, int seq, int sseq, float c2, int64_t b,
                                               int rb, int k0, int keys, _Float16* ldsQ, int64_t& qrow) {
     float* lbias = reinterpret_cast<float*>(ldsQ + 2 * kPanelHalvesQ<D>);  // this key range's bias
     const int tid = threadIdx.x;
@@ -166,18 +173,19 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
     const int np = keys / kPanelQ;
     qrow = b * seq + static_cast<int64_t>(rb) * 128 + wave * 32 + l32;
     constexpr int KS = D / 16;
+    const _Float16* qr = Q + (RAGGED ? b * sseq + min(rb * 128 + wave * 32 + l32, sseq - 1) : qrow) * D;
     f16x8 xq[KS];                                 // B operand: this lane's query, KS x 16 head dims
 #pragma unroll
-    for (int ks = 0; ks < KS; ++ks) xq[ks] = *reinterpret_cast<const f16x8*>(Q + qrow * D + ks * 16 + hl * 8);
-    for (int i = tid; i < keys; i += 256) lbias[i] = biasLog2(bias[k0 + i]);
-    const _Float16* kb = K + (b * seq + k0) * D;
+    for (int ks = 0; ks < KS; ++ks) xq[ks] = *reinterpret_cast<const f16x8*>(qr + ks * 16 + hl * 8);
+    for (int i = tid; i < keys; i += 256) lbias[i] = RAGGED && k0 + i >= sseq ? -INFINITY : biasLog2(bias[k0 + i]);
+    const _Float16* kb = K + b * (RAGGED ? sseq : seq) * D;
     u32x4v v[D / 16];
-    loadPanelQ<D>(kb, tid, v);
+    loadPanelQ<D, RAGGED>(kb, k0, sseq, tid, v);
     storePanelQ<D>(ldsQ, tid, v);
     __syncthreads();
     float m = -INFINITY, l = 0.0f;
     for (int p = 0; p < np; ++p) {
-        if (p + 1 < np) loadPanelQ<D>(kb + static_cast<int64_t>(p + 1) * kPanelQ * D, tid, v);
+        if (p + 1 < np) loadPanelQ<D, RAGGED>(kb, k0 + (p + 1) * kPanelQ, sseq, tid, v);
         const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ<D>;
         f32x16 acc[4];
 #pragma unroll
@@ -268,9 +276,8 @@ __device__ __forceinline__ bool mergeStatsQ(const float2 (&pp)[kMaxRangesQ], int
 
 /// Pass 2 over keys [k0, k0 + keys) of this wave's 32 rows r0..r0+31 of
 /// batch b: D = Q K^T per panel, written as exp2(v - shift) * scale at once.
-/// RAGGED: Q, K and the bias are zero-padded copies of length seq of a sequence
-/// of length sseq; S is [batch][sseq][sseq] and only rows and keys below sseq
-/// are stored. QUADS (S 16-byte aligned, sseq a multiple of 4): MFMA column l
+/// RAGGED: seq is the sequence length sseq of the operands rounded up to whole
+/// panels; what is past its end repeats its last row and is not stored. QUADS (S 16-byte aligned, sseq a multiple of 4): MFMA column l
 /// of block j is key 4 l + j, so that a lane's four blocks hold four keys in a
 /// row and one store writes 512 bytes of each of two rows (8 x 1024 x 64: 15.1
 /// -> 13.9 us against 128 bytes); otherwise it is key 32 j + l and a store
@@ -290,12 +297,13 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
     const int lane = tid & 63, l32 = lane & 31, hl = lane >> 5;
     const int np = keys / kPanelQ;
     constexpr int KS = D / 16;
+    const _Float16* qr = Q + (RAGGED ? b * ld + min(i0 + l32, ld - 1) : r0 + l32) * D;
     f16x8 aq[KS];                                 // A operand: row r0 + l32
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) {
-        aq[ks] = *reinterpret_cast<const f16x8*>(Q + (r0 + l32) * D + ks * 16 + hl * 8);
+        aq[ks] = *reinterpret_cast<const f16x8*>(qr + ks * 16 + hl * 8);
     }
-    const _Float16* kb = K + (b * seq + k0) * D;
+    const _Float16* kb = K + b * ld * D;
     // Stores: a scalar base per panel (row r0, key kc) plus a fixed lane
     // offset per accumulator register r.
     const int lk = QUADS ? 4 * l32 : l32;         // this lane's key of block 0
@@ -310,7 +318,7 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
     for (int i = 0; i < kMaxRangesQ; ++i) pp[i] = part[(r0 + l32) * nr + (i < nr ? i : 0)];
     u32x4v v[D / 16];
     int at = static_cast<int>(b) % np;
-    loadPanelQ<D>(kb + static_cast<int64_t>(at) * kPanelQ * D, tid, v);
+    loadPanelQ<D, RAGGED>(kb, k0 + at * kPanelQ, ld, tid, v);
     float shift[16], scale[16];
     const bool plain = mergeStatsQ(pp, nr, shift, scale);
     storePanelQ<D, QUADS>(ldsQ, tid, v);
@@ -318,7 +326,7 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
     for (int p = 0; p < np; ++p) {
         const int kc = k0 + at * kPanelQ;
         if (++at == np) at = 0;
-        if (p + 1 < np) loadPanelQ<D>(kb + static_cast<int64_t>(at) * kPanelQ * D, tid, v);
+        if (p + 1 < np) loadPanelQ<D, RAGGED>(kb, k0 + at * kPanelQ, ld, tid, v);
         const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ<D>;
         f32x16 acc[4];
 #pragma unroll
@@ -336,7 +344,7 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
         }
         float bj[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bj[j] = biasLog2(bias[kc + lk + j * jk]);
+        for (int j = 0; j < 4; ++j) bj[j] = biasLog2(bias[RAGGED ? min(kc + lk + j * jk, ld - 1) : kc + lk + j * jk]);
         char* sb = reinterpret_cast<char*>(S + (b * ld + i0) * static_cast<int64_t>(ld) + kc);
         auto store = [&](auto value) {
 #pragma unroll
@@ -365,17 +373,18 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
     }
 }
 
-template <int D>
+template <int D, bool RAGGED>
 __global__ __launch_bounds__(256, 2) void scoreStatsQ(const _Float16* __restrict__ Q,
                                                       const _Float16* __restrict__ K,
                                                       const float* __restrict__ bias,
-                                                      float2* __restrict__ part, int seq, int nr, int per, float c2) {
+                                                      float2* __restrict__ part, int seq, int sseq, int nr, int per,
+                                                      float c2) {
     extern __shared__ __align__(16) _Float16 ldsQ[];
     int64_t b;
     int rb, kr, k0, keys;
     blockOfQ(seq, nr, per, b, rb, kr, k0, keys);
     int64_t qrow;
-    const float2 st = statsRangeQ<D>(Q, K, bias, seq, c2, b, rb, k0, keys, ldsQ, qrow);
+    const float2 st = statsRangeQ<D, RAGGED>(Q, K, bias, seq, sseq, c2, b, rb, k0, keys, ldsQ, qrow);
     if (((threadIdx.x & 63) >> 5) == 0) part[qrow * nr + kr] = st;
 }
 
@@ -422,23 +431,33 @@ int rangesQ(const mlkd_score_softmax* p, int most = kMaxRangesQ) {
     return static_cast<int>((p->seq / kPanelQ + per - 1) / per);
 }
 
-/// Both passes over p's (padded) Q, K and bias, at most `most` key ranges per
-/// row block with their partials in p->scratch; `ragged` > 0 stores only rows and keys
-/// below it into p->s laid out [batch][ragged][ragged].
+/// Both passes, at most `most` key ranges per row block with their partials in
+/// p->scratch; `ragged` > 0 is the operands' sequence length, p->seq that
+/// rounded up to whole panels. Copies of Q, K and the bias, padded by three
+/// kernels more, took 16 x 1000 x 128 to 33 us (24 without), 4 x 1000 to 19
+/// (12.7), 1 x 300 to 21 (9.9).
 template <int D>
-int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragged) {
+int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragged = 0) {
+    auto stats = scoreStatsQ<D, false>;
+    auto storeAny = scoreStoreQ<D, true, false>, store = scoreStoreQ<D, false, true>;
     // Once per process; a function-local static initializes thread-safely.
-    static const bool attrs = [] {
-        const int maxStats = static_cast<int>(kLdsStoreQ<D> + static_cast<size_t>(kMaxSeqQ) * sizeof(float));
-        for (const void* fn : {reinterpret_cast<const void*>(scoreStatsQ<D>),
-                               reinterpret_cast<const void*>(scoreStoreQ<D, false, true>),
-                               reinterpret_cast<const void*>(scoreStoreQ<D, true, true>),
-                               reinterpret_cast<const void*>(scoreStoreQ<D, true, false>)}) {
-            if (hipFuncSetAttribute(fn, hipFuncAttributeMaxDynamicSharedMemorySize, maxStats) != hipSuccess) return false;
-        }
-        return true;
-    }();
+    auto allow = [](auto fn) {
+        const int bytes = static_cast<int>(kLdsStoreQ<D> + static_cast<size_t>(kMaxSeqQ) * sizeof(float));
+        return hipFuncSetAttribute(reinterpret_cast<const void*>(fn), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                   bytes) == hipSuccess;
+    };
+    static const bool attrs = allow(stats) && allow(store) && allow(storeAny);
     if (!attrs) return MLKD_RT_LAUNCH;
+    if constexpr (D == 128) {   // dim 64 is not run off the panels
+        static const bool raggedAttrs = allow(scoreStatsQ<D, true>) && allow(scoreStoreQ<D, true, true>);
+        if (!raggedAttrs) return MLKD_RT_LAUNCH;
+        if (ragged > 0) {
+            stats = scoreStatsQ<D, true>;
+            store = scoreStoreQ<D, true, true>;
+        }
+    }
+    const int64_t sseq = ragged > 0 ? ragged : p->seq;
+    if (sseq % 4 != 0 || (reinterpret_cast<uintptr_t>(p->s) & 15u) != 0) store = storeAny;
     const int per = panelsPerRange(p, most) * kPanelQ;
     const size_t ldsStats = kLdsStoreQ<D> + static_cast<size_t>(per) * sizeof(float);
     const int nr = rangesQ(p, most);
@@ -446,14 +465,10 @@ int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragge
     // Both passes work in base 2: v2 = acc * (log2(e) / div) + bias * log2(e),
     // exp(v - max) = exp2(v2 - max2).
     const float c2 = static_cast<float>(1.4426950408889634 / p->div);
-    hipLaunchKernelGGL(scoreStatsQ<D>, grid, dim3(256), ldsStats, st, static_cast<const _Float16*>(p->q),
+    hipLaunchKernelGGL(stats, grid, dim3(256), ldsStats, st, static_cast<const _Float16*>(p->q),
                        static_cast<const _Float16*>(p->k), static_cast<const float*>(p->bias),
-                       static_cast<float2*>(p->scratch), static_cast<int>(p->seq), nr, per, c2);
-    const int64_t sseq = ragged > 0 ? ragged : p->seq;
-    auto store = scoreStoreQ<D, true, false>;
-    if (sseq % 4 == 0 && (reinterpret_cast<uintptr_t>(p->s) & 15u) == 0) {
-        store = ragged > 0 ? scoreStoreQ<D, true, true> : scoreStoreQ<D, false, true>;
-    }
+                       static_cast<float2*>(p->scratch), static_cast<int>(p->seq),
+                       static_cast<int>(sseq), nr, per, c2);
     hipLaunchKernelGGL(store, grid, dim3(256), kLdsStoreQ<D>, st,
                        static_cast<const _Float16*>(p->q), static_cast<const _Float16*>(p->k),
                        static_cast<const float*>(p->bias), static_cast<const float2*>(p->scratch),
@@ -513,55 +528,22 @@ __global__ __launch_bounds__(256) void scoresGeneral(mlkd_score_softmax p) {
     }
 }
 
-/// [batch][rows][128] f16 -> [batch][drows][128], zero rows past `rows`, in
-/// 16-byte pieces (16 per row).
-__global__ __launch_bounds__(256) void padQK(const u32x4v* __restrict__ src, int64_t batch, int64_t rows,
-                                             u32x4v* __restrict__ dst, int64_t drows) {
-    const int64_t total = batch * drows * 16;
-    for (int64_t t = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; t < total;
-         t += static_cast<int64_t>(gridDim.x) * 256) {
-        const int64_t piece = t & 15, r = t >> 4;
-        const int64_t b = r / drows, i = r % drows;
-        dst[t] = i < rows ? src[(b * rows + i) * 16 + piece] : u32x4v{0u, 0u, 0u, 0u};
-    }
-}
-
-/// bias' = bias on [0, seq), -inf on [seq, dseq): padded keys take no share.
-__global__ __launch_bounds__(256) void padBias(const float* __restrict__ src, int64_t seq, float* __restrict__ dst,
-                                               int64_t dseq) {
-    for (int64_t j = static_cast<int64_t>(blockIdx.x) * 256 + threadIdx.x; j < dseq;
-         j += static_cast<int64_t>(gridDim.x) * 256) {
-        dst[j] = j < seq ? src[j] : -INFINITY;
-    }
-}
-
-/// Workspace bytes of the two passes: nothing but the partials where p's
-/// sequence is whole panels, otherwise copies of Q, K and the bias padded to a
-/// whole number first. 0 where the two passes don't run on a workspace.
-/// `q`, if given, is set up to run in the workspace p->work.
+/// Workspace bytes of the two passes, for their partials: 0 where they don't
+/// run. `q`, if given, is p over whole panels, set up to run in the workspace
+/// p->work.
 int64_t workBytes(const mlkd_score_softmax* p, mlkd_score_softmax* q = nullptr) {
     mlkd_score_softmax w = *p;
     w.seq = (p->seq + kPanelQ - 1) / kPanelQ * kPanelQ;
-    if (!twoPassApplies(&w)) return 0;
-    int64_t at = 0;
-    unsigned char* base = static_cast<unsigned char*>(p->work);
-    if (w.seq != p->seq) {
-        // Off the panels at dim 64 the general kernels run.
-        if (p->dim != 128) return 0;
-        const int64_t qk = p->batch * w.seq * p->dim * static_cast<int64_t>(sizeof(_Float16));
-        w.q = base;
-        w.k = base + qk;
-        w.bias = base + 2 * qk;
-        at = 2 * qk + w.seq * static_cast<int64_t>(sizeof(float));
-    }
-    w.scratch = base + at;
+    // Off the panels the general kernels, which add in f64, run dim 64.
+    if (!twoPassApplies(&w) || (w.seq != p->seq && p->dim != 128)) return 0;
+    w.scratch = p->work;
     w.scratch_bytes = statsBytes(&w, rangesQ(&w));
     if (q != nullptr) *q = w;
-    return at + w.scratch_bytes;
+    return w.scratch_bytes;
 }
 
 /// Scratch a run of the two passes is always given: dim 128, whole pairs of
-/// panels, two key ranges. Elsewhere, and for more ranges, they take a
+/// panels, for two key ranges. Elsewhere, and for more ranges, they take a
 /// workspace where there is one.
 int64_t requiredBytes(const mlkd_score_softmax* p) {
     return p->dim == 128 && p->seq % (2 * kPanelQ) == 0 && twoPassApplies(p) ? statsBytes(p, 2) : 0;
@@ -587,22 +569,7 @@ bool runsTwoPass(const mlkd_score_softmax* p, int variant, mlkd_score_softmax& q
 
 int launchTwoPass(const mlkd_score_softmax* p, const mlkd_score_softmax& q, int most, hipStream_t st) {
     const int64_t ragged = q.seq == p->seq ? 0 : p->seq;
-    if (ragged > 0) {
-        // Copies padded with zero rows and -inf bias, and both passes over
-        // them, are faster than the general kernels at every size measured,
-        // down to 1 x 100 x 128 (general: 41 us).
-        const int64_t pieces = p->batch * q.seq * 16;
-        const unsigned g = static_cast<unsigned>(std::min<int64_t>((pieces + 255) / 256, 16384));
-        hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->q), p->batch, p->seq,
-                           static_cast<u32x4v*>(const_cast<void*>(q.q)), q.seq);
-        hipLaunchKernelGGL(padQK, dim3(g), dim3(256), 0, st, static_cast<const u32x4v*>(p->k), p->batch, p->seq,
-                           static_cast<u32x4v*>(const_cast<void*>(q.k)), q.seq);
-        hipLaunchKernelGGL(padBias, dim3(static_cast<unsigned>((q.seq + 255) / 256)), dim3(256), 0, st,
-                           static_cast<const float*>(p->bias), p->seq, static_cast<float*>(const_cast<void*>(q.bias)),
-                           q.seq);
-        if (hipGetLastError() != hipSuccess) return MLKD_RT_LAUNCH;
-    }
-    return p->dim == 64 ? launchQ<64>(&q, most, st, ragged) : launchQ<128>(&q, most, st, ragged);
+    return p->dim == 64 ? launchQ<64>(&q, most, st) : launchQ<128>(&q, most, st, ragged);
 }
 
 // 0: the best form for the shape (the two-pass query-stationary form where

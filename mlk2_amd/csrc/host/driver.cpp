@@ -459,8 +459,8 @@ int HipLoadedKernel::arenaLayout(const DeviceBinding* binds, int64_t elements, c
         return MLKHIP_REFUSED;
     }
     // Workspaces a step can do without (aligned copies of a GEMM's operands
-    // or the sums of its K ranges, score-softmax statistics and padded copies)
-    // take the room that is left, in step order; a step whose workspace does
+    // or the sums of its K ranges, score-softmax statistics) take the room that
+    // is left, in step order; a step whose workspace does
     // not fit runs on the kernels that need none.
     padOff.assign(plan_.steps.size(), SIZE_MAX);
     for (size_t si = 0; si < plan_.steps.size(); ++si) {

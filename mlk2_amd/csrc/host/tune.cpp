@@ -425,7 +425,7 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
             perGroup = ranges > 0 ? (128 * sp + ranges - 1) / ranges : 64 * 128;
             covered = workgroups * perGroup >= instances;
             form = ranges == 0     ? "64 x 128 score tiles, then row softmax"
-                   : sp != st.seq  ? "128-row blocks x key ranges, per pass, over zero-padded Q and K"
+                   : sp != st.seq  ? "128-row blocks x key ranges, per pass, bounded by the sequence"
                                    : "128-row blocks x key ranges, per pass";
             break;
         }
