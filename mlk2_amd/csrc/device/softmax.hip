@@ -605,7 +605,8 @@ bool wideApplies(const mlkd_softmax* p) {
     const bool f32 = p->x_dtype == MLKD_F32 && p->y_dtype == MLKD_F32;
     const bool f16 = p->x_dtype == MLKD_F16 && p->y_dtype == MLKD_F16;
     const int64_t es = f32 ? 4 : 2;
-    return (f32 || f16) && p->cols >= 16 && p->cols >= 16 && p->rows <= 0x7FFFFFFF && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->cols >= 16 && p->x_row_stride == p->y_row_stride && p->cols <= 65536 &&
+    return (f32 || f16) && p->rows <= 0x7FFFFFFF && p->cols >= 16 && p->cols <= 65536 &&
+           p->x_row_stride == p->y_row_stride &&
            ((reinterpret_cast<uintptr_t>(p->x) ^ reinterpret_cast<uintptr_t>(p->y)) & 15u) == 0 &&
            reinterpret_cast<uintptr_t>(p->x) % static_cast<uintptr_t>(es) == 0;
 }
