@@ -231,6 +231,7 @@ void HipLoadedKernel::freeScratch(RunScratch& rs) {
     for (void* p : rs.step) {
         if (p != nullptr) mlkd_rt_free(p);
     }
+    for (void* p : rs.outgrown) mlkd_rt_free(p);
 }
 
 HipLoadedKernel::~HipLoadedKernel() {
@@ -281,14 +282,17 @@ int64_t HipLoadedKernel::stepScratch(RunScratch& rs, size_t si, int64_t need, in
     void*& p = rs.step[si];
     int64_t& bytes = rs.stepBytes[si];
     if (bytes < (need > 0 ? need : want)) {
-        if (p != nullptr) mlkd_rt_free(p);
-        bytes = 0;
-        if (want > need && mlkd_rt_malloc_spare(&p, static_cast<size_t>(want), stream) == 0) {
-            bytes = want;
-        } else if (need > 0 && mlkd_rt_malloc(&p, static_cast<size_t>(need)) == 0) {
-            bytes = need;
-        } else {
-            p = nullptr;
+        void* block = nullptr;
+        int64_t size = 0;
+        if (want > need && mlkd_rt_malloc_spare(&block, static_cast<size_t>(want), stream) == 0) {
+            size = want;
+        } else if (need > 0 && mlkd_rt_malloc(&block, static_cast<size_t>(need)) == 0) {
+            size = need;
+        }
+        if (size > 0) {
+            if (p != nullptr) rs.outgrown.push_back(p);
+            p = block;
+            bytes = size;
         }
     }
     *ptr = p;

@@ -114,12 +114,15 @@ private:
         void* status{nullptr};
         std::vector<void*> step;
         std::vector<int64_t> stepBytes;
+        std::vector<void*> outgrown;   // smaller blocks of `step`: a captured graph may still use them
     };
     RunScratch& scratchFor(void* stream) const;  // caller holds scratchLock_
     static void freeScratch(RunScratch& rs);
     /// Bytes of rs.step[si] (at *ptr), allocated on first use: `want` where the step can
     /// do without it and they can be had (not while `stream` is captured),
-    /// otherwise `need`; less than that when the allocation fails.
+    /// otherwise `need`; less than that when the allocation fails. A GEMM's
+    /// `want` varies with the alignment of its operands (copies of A, of B or
+    /// of both), so a step outgrows at most two blocks.
     int64_t stepScratch(RunScratch& rs, size_t si, int64_t need, int64_t want, void* stream, void** ptr) const;
     /// Offsets of a run's scratch in `arena`; refuses what does not fit or
     /// needs a host read-back.

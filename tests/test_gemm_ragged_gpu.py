@@ -11,6 +11,7 @@ import pytest
 import oracle
 from mlk2_amd import fixtures as fx
 from mlk2_amd.backend import Binding, DeviceBuffer
+from test_score_two_pass_gpu import _Capture
 
 pytestmark = pytest.mark.gpu
 NP = {"f16": np.float16, "f32": np.float32}
@@ -111,3 +112,33 @@ def test_allocation_free_entry_without_room(hip):
     y = DeviceBuffer(m * n, "f32")
     art.run_device_noalloc({0: ab, 1: bb, 2: y})
     check(y.to_numpy(), a, b, c, False)
+
+
+def test_captured_workspace_outlives_a_larger_one(hip):
+    # A graph holds the workspace of A's copy; a run that copies B too asks for
+    # a larger one, and the graph's stays until the artifact is released.
+    m, k, n = 300, 104, 264
+    a, b, c = operands(m, k, n, "f16")
+    art = hip.build(module(m, k, n, "f16", False))
+    off, even, odd = _At(a, "f16", 1), _At(b, "f16", 0), _At(b, "f16", 3)
+    out, eager = DeviceBuffer(m * n, "f32"), DeviceBuffer(m * n, "f32")
+    cap = _Capture()
+    stream = cap.stream.value
+
+    def run(bound, y):
+        art.run_device({0: off, 1: bound, 2: y}, stream=stream, sync=False)
+        cap("hipStreamSynchronize", cap.stream)
+        check(y.to_numpy(), a, b, c, False)
+
+    run(even, eager)
+    with cap:
+        art.run_device({0: off, 1: even, 2: out}, stream=stream, sync=False)
+    run(odd, eager)
+    others = [DeviceBuffer.from_array(np.full(m * 128, 3.0), "f16") for _ in range(8)]
+    for bound in (odd, even, odd):
+        cap.replay()
+        check(out.to_numpy(), a, b, c, False)
+        run(bound, eager)
+    for other in others:
+        assert (other.to_numpy() == 3.0).all()
+    cap.close()
