@@ -60,6 +60,16 @@ def test_edges(hip, dtype, m, k, n, call):
     check(got, a, b, c, dtype, call)
 
 
+# Each XCD's share of the tiles, where 8 do not divide them: every tile once.
+@pytest.mark.parametrize("tiles", [1, 7, 8, 9, 15, 17, 22, 27])
+@pytest.mark.parametrize("m", [16, 40])
+def test_numbers_of_tiles(hip, m, tiles):
+    a, b, c = operands(m, 40, 32 * tiles - 1, "f64")
+    got = hip.build(module(m, 40, 32 * tiles - 1, "f64", True)).run(
+        {0: a.reshape(-1), 1: b.reshape(-1), 2: c.reshape(-1)})[2]
+    check(got, a, b, c, "f64", True)
+
+
 def test_names(hip):
     # Long K over few tiles: K ranges in several workgroups, then their sum.
     name = hip.build(module(16, 4096, 4096, "f16", False)).step_kernel_name(0)
