@@ -338,14 +338,16 @@ struct WideRow<_Float16> {
 
 /// softmaxRowWide's row for a max that is infinite or so large that floats
 /// near it lie far apart (or, in f16, end): the same arithmetic, element by
-/// element from memory, with the exponent itself held at -1000 or more. x and
-/// y may be the same row: each element is read before its thread writes it.
+/// element from memory, with the exponent itself held at -1000 or more. The
+/// max is subtracted before the scale: x * log2(e) + round(-m * log2(e)) is off
+/// at x == m by the product's rounding, which leaves [-1000, 1000] from |m| of
+/// 1e20 on. x and y may be the same row: each element is read before its
+/// thread writes it.
 template <typename T, int W>
 __device__ __forceinline__ void softmaxOddRow(const T* x, T* y, int cols, float m, int thread, double (&slot)[W]) {
     using R = WideRow<T>;
-    const double mb = static_cast<double>(m) * -1.4426950408889634074;
     auto term = [&](T xv) {
-        const double e = __builtin_fma(static_cast<double>(static_cast<float>(xv)), 1.4426950408889634074, mb);
+        const double e = (static_cast<double>(static_cast<float>(xv)) - static_cast<double>(m)) * 1.4426950408889634074;
         return exp2Poly(e < -1000.0 ? -1000.0 : e, kExp2C10);
     };
     double s = 0.0;

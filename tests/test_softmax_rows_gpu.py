@@ -71,6 +71,29 @@ def test_scalar_rows_over_four_waves(hip, n):
     check(art.run({0: x.reshape(-1)})[1], x, "f32", tight=False)
 
 
+def large_rows(n):
+    """Finite maxima from where exp's arguments need more than 53 bits of x *
+    log2(e) up to the largest float, of either sign, and constant rows."""
+    x = np.zeros((13, n), np.float32)
+    for r, v in enumerate([1e7, 1e19, 1e20, 1e25, 1e30, np.finfo(np.float32).max]):
+        x[r, n // 3] = v
+        x[6 + r] = -2.0 * v if v < 1e38 else -v
+        x[6 + r, n - 1] = -v if v < 1e38 else -v / 2
+    x[12] = np.float32(2.0 ** 84)
+    return x
+
+
+@pytest.mark.parametrize("n,skip", [(9000, 0), (9000, 3), (20000, 0), (65536, 0)])
+@pytest.mark.parametrize("in_place", [False, True])
+def test_rows_of_large_values(hip, n, skip, in_place):
+    x = large_rows(n)
+    art = hip.build(fx.softmax_call_module(*x.shape, "f32"))
+    xb = _At(x, "f32", skip)
+    yb = xb if in_place else _At(np.zeros_like(x), "f32", skip)
+    art.run_device({0: xb, 1: yb})
+    check(yb.values(), x, "f32")
+
+
 class _At:
     """A device buffer bound `skip` elements into its allocation."""
 
