@@ -82,6 +82,19 @@ def test_non_finite_columns_skip_zeros(hip, dtype, m, k, n):
     assert (np.abs(part[fin] - ref[fin]) <= ((k + 3) * (U + 2.0 ** -53) * (size + np.abs(c[rows])))[fin]).all()
 
 
+# One infinity in B: 15 times the finite product's time (206, with one row and
+# one step's loads at a time).
+def test_non_finite_products_stay_fast(hip):
+    n = 1000
+    a, b, c = operands(n, n, n, "f32")
+    art = hip.build(module(n, n, n, "f32", True))
+    bufs = {0: DeviceBuffer.from_array(a, "f32"), 1: DeviceBuffer.from_array(b, "f32"), 2: DeviceBuffer.from_array(c, "f32")}
+    finite = art.time_device_span(bufs, 10)
+    b[n // 2, n // 3] = np.inf
+    bufs[1] = DeviceBuffer.from_array(b, "f32")
+    assert art.time_device_span(bufs, 3, 1) <= 60 * finite
+
+
 class _At:
     def __init__(self, x, dtype, skip):
         pad = np.zeros(skip + x.size + 8, NP[dtype])
