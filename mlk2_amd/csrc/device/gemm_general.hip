@@ -194,16 +194,40 @@ struct Direct<double> {
     }
 };
 
+/// 16 bytes of consecutive elements at any element alignment.
+template <typename T>
+struct __attribute__((packed, aligned(sizeof(T)))) Packed {
+    typename Direct<T>::Vec v;
+};
+
 /// Call(MatMul)'s element, as the reference computes it: C_in plus A[i,p] *
 /// B[p,j] over p ascending, skipping A[i,p] == 0. The skip changes an element
 /// only where its column of B holds an infinity or a NaN, and there the
-/// MFMA sum is not finite (0 * inf is NaN), so only such elements take this.
+/// MFMA sum is not finite (0 * inf is NaN), so only such elements take this,
+/// or exactTile. The sum is one serial chain, so 16 steps' loads go out ahead
+/// of it (16x4096x1024 f64 with one infinity in B: 147 us; one step at a time
+/// 1249).
 template <typename T, typename O>
 __device__ __forceinline__ O exactElement(const T* a, const T* b, int64_t ldb, int k, O c) {
-    for (int p = 0; p < k; ++p) {
-        const O av = static_cast<O>(a[p]);
-        if (av != O(0)) c = c + av * static_cast<O>(b[p * ldb]);
+    constexpr int V = Direct<T>::V, U = 16;
+    auto step = [&](T at, T bt) {
+        const O av = static_cast<O>(at);
+        if (av != O(0)) c = c + av * static_cast<O>(bt);
+    };
+    int p = 0;
+#pragma unroll 1
+    for (; p + U <= k; p += U) {
+        typename Direct<T>::Vec av[U / V];
+        T bv[U];
+#pragma unroll
+        for (int i = 0; i < U / V; ++i) av[i] = reinterpret_cast<const Packed<T>*>(a + p + i * V)->v;
+#pragma unroll
+        for (int i = 0; i < U; ++i) bv[i] = b[(p + i) * ldb];
+#pragma unroll
+        for (int i = 0; i < U; ++i) step(av[i / V][i % V], bv[i]);
     }
+#pragma unroll 1
+    for (; p < k; ++p) step(a[p], b[p * ldb]);
     return c;
 }
 
@@ -222,11 +246,59 @@ struct DirectArgs {
     int accumulate, skip;
 };
 
-/// 16 bytes of consecutive elements at any element alignment.
-template <typename T>
-struct __attribute__((packed, aligned(sizeof(T)))) Packed {
-    typename Direct<T>::Vec v;
-};
+/// exactElement over a workgroup's whole tile, up to R rows of a column to a
+/// thread, K by slabs of KC through LDS. Measured with one infinity in B (each
+/// element by itself, one step at a time; the scalar kernel): f64 512^3 84 us
+/// (195; 163), 1024^3 308 us (1714; 372).
+template <typename T, int MT>
+__device__ __forceinline__ void exactTile(const DirectArgs<T, MT>& p, int row0, int col0, unsigned char* lds) {
+    using Out = typename Direct<T>::Out;
+    constexpr int R = MT == 1 ? 4 : 8, KC = 8, TR = 16 * MT, TC = 16 * Direct<T>::V;
+    static_assert(KC * (TR + TC) * sizeof(T) <= MT * Direct<T>::V * 64 * sizeof(typename Direct<T>::Acc),
+                  "the slabs fit the sums' LDS");
+    T* as = reinterpret_cast<T*>(lds);   // [KC][TR]
+    T* bs = as + KC * TR;                // [KC][TC]
+    const int rows = min(TR, p.m - row0), cols = min(TC, p.n - col0);
+    const int tid = static_cast<int>(threadIdx.x), threads = 64 * p.waves;
+    const int cw = min(TC, threads), step = threads / cw;   // columns at once; rows apart of a thread's
+    for (int cb = 0; cb < cols; cb += cw) {
+        for (int rb = 0; rb < rows; rb += R * step) {
+            const int col = cb + tid % cw, row = rb + tid / cw;
+            const int staged = min(R * step, TR - rb);
+            Out* c = p.c + static_cast<int64_t>(row0) * p.ldc + col0 + col;
+            Out s[R];
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                s[i] = col < cols && row + i * step < rows ? c[(row + i * step) * p.ldc] : Out(0);
+            }
+            for (int k0 = 0; k0 < p.k; k0 += KC) {
+                __syncthreads();
+                for (int e = tid; e < staged * KC; e += threads) {
+                    const int r = rb + e / KC, k = k0 + e % KC;
+                    as[e % KC * TR + e / KC] = r < rows && k < p.k ? p.a[(row0 + r) * p.lda + k] : T(0);
+                }
+                for (int e = tid; e < cw * KC; e += threads) {
+                    const int k = k0 + e / cw, j = cb + e % cw;
+                    bs[e / cw * TC + e % cw] = j < cols && k < p.k ? p.b[k * p.ldb + col0 + j] : T(0);
+                }
+                __syncthreads();
+#pragma unroll
+                for (int k = 0; k < KC; ++k) {
+                    const Out bv = static_cast<Out>(bs[k * TC + tid % cw]);
+#pragma unroll
+                    for (int i = 0; i < R; ++i) {
+                        const Out av = static_cast<Out>(as[k * TR + min(tid / cw + i * step, TR - 1)]);
+                        if (av != Out(0)) s[i] = s[i] + av * bv;
+                    }
+                }
+            }
+#pragma unroll
+            for (int i = 0; i < R; ++i) {
+                if (col < cols && row + i * step < rows) c[(row + i * step) * p.ldc] = s[i];
+            }
+        }
+    }
+}
 
 /// One tile, operands straight from global memory into MFMA operand registers
 /// (the layouts above make every load 16 bytes of a row), so that a small
@@ -351,38 +423,66 @@ __device__ __forceinline__ void directTile(const DirectArgs<T, MT>& p) {
         }
         __syncthreads();
     }
+    Out* part = gridDim.y > 1 ? p.part + static_cast<int64_t>(blockIdx.y) * p.m * p.n : nullptr;
+    const bool exact = p.skip && part == nullptr;   // a sum that is not finite: exactTile
+    int* odd = reinterpret_cast<int*>(red + 64);    // in the spare entries
     if (wave == 0) {
+        bool bad = false;
 #pragma unroll
         for (int t = 0; t < MT; ++t) {
 #pragma unroll
-            for (int j = 0; j < V; ++j) *slot(0, t, j) = acc[t][j];
+            for (int j = 0; j < V; ++j) {
+                *slot(0, t, j) = acc[t][j];
+#pragma unroll
+                for (int e = 0; e < 4; ++e) bad |= exact && !__builtin_isfinite(acc[t][j][e]);
+            }
+        }
+        if (exact) {
+            const bool any = __builtin_amdgcn_ballot_w64(bad) != 0;
+            if (lane == 0) *odd = any ? 1 : 0;
         }
     }
     __syncthreads();
+    if (__builtin_expect(exact && __builtin_amdgcn_readfirstlane(*odd) != 0, 0)) {   // out of the cold path
+        exactTile<T, MT>(p, row0, col0, ldsG);
+        return;
+    }
     const Out* sums = reinterpret_cast<const Out*>(ldsG);
     const int rows = min(16 * MT, p.m - row0), cols = min(16 * V, p.n - col0);
-    Out* part = gridDim.y > 1 ? p.part + static_cast<int64_t>(blockIdx.y) * p.m * p.n : nullptr;
     // Column i of the tile is column i - shift of the ones read (shift > 0
     // in the last lane read of a ragged N: its V columns end at N).
-    for (int i = static_cast<int>(threadIdx.x); i < rows * (16 * V); i += 64 * p.waves) {
-        const int row = i / (16 * V), col = i % (16 * V);
-        if (col >= cols) continue;
+    auto sumAt = [&](int row, int col) {
         const int owner = col / V;
         const int j = col0 + col - min(col0 + owner * V, p.n - V);
         const int q = row % 16;
-        const int from = (((row / 16) * V + j) * F + D::group(q) * 16 + owner) * 4 + D::entry(q);
-        Out v = sums[from];
-        if (part != nullptr) {
-            part[static_cast<int64_t>(row0 + row) * p.n + col0 + col] = v;
-            continue;
+        return sums[(((row / 16) * V + j) * F + D::group(q) * 16 + owner) * 4 + D::entry(q)];
+    };
+    const int threads = 64 * p.waves;
+    if (p.accumulate && part == nullptr) {
+        // Four rows of C read before the first is written (one: f16
+        // 200x700x300 with C += A B 7.5 us, four: 6.8).
+        constexpr int R = 4;
+        const int cw = min(16 * V, threads), step = threads / cw;
+        for (int col = static_cast<int>(threadIdx.x) % cw; col < cols; col += cw) {
+            for (int row = static_cast<int>(threadIdx.x) / cw; row < rows; row += R * step) {
+                Out* dst = p.c + static_cast<int64_t>(row0 + row) * p.ldc + col0 + col;
+                Out v[R];
+#pragma unroll
+                for (int i = 0; i < R; ++i) v[i] = row + i * step < rows ? dst[i * step * p.ldc] : Out(0);
+#pragma unroll
+                for (int i = 0; i < R; ++i) {
+                    if (row + i * step < rows) dst[i * step * p.ldc] = v[i] + sumAt(row + i * step, col);
+                }
+            }
         }
-        Out* dst = p.c + static_cast<int64_t>(row0 + row) * p.ldc + col0 + col;
-        const Out old = p.accumulate ? *dst : Out(0);
-        v = old + v;
-        if (p.skip && !__builtin_isfinite(v)) {
-            v = exactElement<T, Out>(p.a + static_cast<int64_t>(row0 + row) * p.lda, p.b + col0 + col, p.ldb, p.k, old);
-        }
-        *dst = v;
+        return;
+    }
+    for (int i = static_cast<int>(threadIdx.x); i < rows * (16 * V); i += threads) {
+        const int row = i / (16 * V), col = i % (16 * V);
+        if (col >= cols) continue;
+        const Out v = sumAt(row, col);
+        if (part != nullptr) part[static_cast<int64_t>(row0 + row) * p.n + col0 + col] = v;
+        else p.c[static_cast<int64_t>(row0 + row) * p.ldc + col0 + col] = v;
     }
 }
 
@@ -421,7 +521,7 @@ __global__ __launch_bounds__(256) void gemmSumParts(DirectArgs<T, 1> p, int rang
 #pragma unroll 8
         for (int s = 1; s < ranges; ++s) v += part[s * total];
         v = old + v;
-        if (p.skip && !__builtin_isfinite(v)) v = exactElement<T, Out>(p.a + row * p.lda, p.b + col, p.ldb, p.k, old);
+        if (__builtin_expect(p.skip && !__builtin_isfinite(v), 0)) v = exactElement<T, Out>(p.a + row * p.lda, p.b + col, p.ldb, p.k, old);
         *dst = v;
     }
 }
