@@ -18,6 +18,7 @@
 // the row with LDS reductions, f64 throughout.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstdio>
 
 #include <math.h>
@@ -607,18 +608,25 @@ bool wideApplies(const mlkd_softmax* p) {
     const bool f32 = p->x_dtype == MLKD_F32 && p->y_dtype == MLKD_F32;
     const bool f16 = p->x_dtype == MLKD_F16 && p->y_dtype == MLKD_F16;
     const int64_t es = f32 ? 4 : 2;
-    return (f32 || f16) && p->rows <= 0x7FFFFFFF && p->cols >= 16 && p->cols <= 65536 &&
+    return (f32 || f16) && p->cols >= 16 && p->cols <= 65536 &&
            p->x_row_stride == p->y_row_stride &&
            ((reinterpret_cast<uintptr_t>(p->x) ^ reinterpret_cast<uintptr_t>(p->y)) & 15u) == 0 &&
            reinterpret_cast<uintptr_t>(p->x) % static_cast<uintptr_t>(es) == 0;
 }
 
+/// A grid holds fewer than 2^32 threads, so fewer than 2^26 rows of one wave
+/// (2 GiB of f16 rows of 16 columns) or 2^24 of four: more go in several
+/// launches of 2^31 threads, whose own time is nothing beside such rows'.
 template <typename T, int CH, int W>
 int launchWideAs(const mlkd_softmax& p, hipStream_t st) {
-    const int64_t blocks = W > 1 ? p.rows : (p.rows + 3) / 4;
-    hipLaunchKernelGGL((softmaxRowWide<T, CH, W>), dim3(static_cast<unsigned>(blocks)), dim3(W == 1 ? 256 : 64 * W), 0,
-                       st, static_cast<const T*>(p.x), static_cast<T*>(p.y), p.rows, static_cast<int>(p.cols),
-                       p.x_row_stride);
+    constexpr int threads = W == 1 ? 256 : 64 * W;
+    constexpr int64_t rowsPer = W > 1 ? 1 : 4, most = (int64_t{1} << 31) / threads * rowsPer;
+    for (int64_t row = 0; row < p.rows; row += most) {
+        const int64_t rows = std::min(p.rows - row, most);
+        hipLaunchKernelGGL((softmaxRowWide<T, CH, W>), dim3(static_cast<unsigned>((rows + rowsPer - 1) / rowsPer)),
+                           dim3(threads), 0, st, static_cast<const T*>(p.x) + row * p.x_row_stride,
+                           static_cast<T*>(p.y) + row * p.x_row_stride, rows, static_cast<int>(p.cols), p.x_row_stride);
+    }
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
 }
 

@@ -12,7 +12,7 @@ import pytest
 
 import oracle
 from mlk2_amd import fixtures as fx
-from mlk2_amd.backend import Binding, DeviceBuffer
+from mlk2_amd.backend import Binding, DeviceBuffer, lib
 
 pytestmark = pytest.mark.gpu
 LOWEST = {"f32": -3.4028234663852886e38, "f16": -65504.0}
@@ -128,3 +128,25 @@ def test_rows_in_place(hip, dtype, n):
     b = DeviceBuffer.from_array(x.reshape(-1), dtype)
     hip.build(fx.softmax_call_module(9, n, dtype)).run_device({0: b, 1: b})
     check(b.to_numpy(), x, dtype)
+
+
+def test_rows_past_one_grid(hip):
+    # 2^26 rows of 16: their workgroups are more threads than one launch holds.
+    m, n = (1 << 26) + 5, 16
+    art = hip.build(fx.softmax_call_module(m, n, "f16"))
+    assert art.step_kernel_name(0).startswith("softmaxRowWide")
+    xb, yb = DeviceBuffer(m * n, "f16"), DeviceBuffer(m * n, "f16")
+    plain = np.tile(np.array([1.0, 2.0], np.float16), n // 2)
+    assert lib().mlkhip_fill32(xb.ptr, int(plain[:2].view(np.uint32)[0]), xb.nbytes) == 0
+    yb.fill_zero()
+    at = [0, 1, (1 << 25) - 1, 1 << 25, (1 << 26) - 1, 1 << 26, m - 1]   # ends of launches and of the rows
+    x = rows_of(len(at), n, "f16")
+    for r, row in zip(at, x):
+        assert lib().mlkhip_memcpy_h2d(xb.ptr + r * n * 2, row.ctypes.data, n * 2) == 0
+    art.run_device({0: xb, 1: yb})
+    got = yb.to_numpy().reshape(m, n)
+    check(got[at], x, "f16")
+    rest = got[2].copy()
+    check(rest, plain.reshape(1, n), "f16")
+    same = (got.view(np.uint64) == rest.view(np.uint64)).all(axis=1)
+    assert same.sum() == m - len(at) and not same[at].any()
