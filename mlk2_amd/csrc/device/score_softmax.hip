@@ -16,6 +16,7 @@
 
 #include <stdint.h>
 
+#include "exp2_poly.h"
 #include "mlk_device_math.h"
 #include "runtime_abi.h"
 #include "xcd.h"
@@ -78,7 +79,7 @@ typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 // MFMAs. At most 73 KiB of LDS and 256 registers per lane let two workgroups
 // share a CU. Scores by 64 x 128 tiles and a softmax over S in place read S
 // back and each K element once per 64 rows: at D 64, 8 x 1024 took 23.5 us
-// and takes 14.4, 16 x 2048 165 and 67.
+// and takes 14.5, 16 x 2048 165 and 72.
 //   Pass 1 (scoreStatsQ) computes D = K Q^T per panel, so each lane holds 64
 //   of its query's scores per panel and keeps a running max and
 //   sum(exp(v - max)) in two registers; the lane 32 away holds the other
@@ -87,8 +88,9 @@ typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 //   Pass 2 (scoreStoreQ) computes D = Q K^T per panel and writes
 //   softmax of the panel at once: each 32-lane half-wave stores
 //   one 128-byte line, while the other workgroup on the CU computes.
-// Both passes work in base 2 with log2(e) folded into 1/div and the bias, so
-// a score costs one fused multiply-add and one v_exp_f32. 16 x 2048 x 128: pass
+// At D 128 both passes work in base 2 with log2(e) folded into 1/div and the
+// bias, so a score costs one fused multiply-add and one v_exp_f32; at D 64 in
+// base e, with f64 sums (StatsQ<64>). 16 x 2048 x 128: pass
 // 1 takes 29 us, bound by its v_exp_f32 (13 us) and MFMAs (7 us), which the
 // two waves of a SIMD overlap in part (panels of 64 keys and four workgroups a
 // CU: no faster); pass 2 takes 45-48 us, bound by its 256 MiB of stores.
@@ -108,11 +110,46 @@ constexpr int64_t kMaxSeqQ = 8192;             // pass 1's LDS stays <= 100 KiB
 /// exp2(-inf - -inf) = NaN; the stored max stays -inf.
 __device__ __forceinline__ float finiteOr0(float m) { return m == -INFINITY ? 0.0f : m; }
 
-/// The bias in base 2. A finite one stays finite, so that keys masked with the
-/// lowest float still share a row that has no others.
-__device__ __forceinline__ float biasLog2(float b) {
+/// The bias in the base of the scores. In base 2 a finite one stays finite, so
+/// that keys masked with the lowest float still share a row that has no others.
+template <int D>
+__device__ __forceinline__ float biasQ(float b) {
+    if (D == 64) return b;
     const float t = b * kLog2e;
     return __builtin_isinf(t) && !__builtin_isinf(b) ? __builtin_copysignf(3.402823466e+38f, t) : t;
+}
+
+/// A row's max and the sum of its weights over one key range.
+template <int D>
+struct StatsQ {
+    float m, l;
+};
+
+/// Head dim 64 keeps the arithmetic of the scores and a softmax over S, its
+/// other form: scores in base e, weights exp2((v - max) * log2(e)), their sum in
+/// f64 by groups of four. In base 2 with f32 sums, as at 128, a row's sum was
+/// off by 5.7e-8 (rms, 8 x 1024; the other form 2.6e-8, so 2.8e-8), and with a
+/// bias of 10 the result by 1.7e-7 (16 x 512; 6.6e-8 and 6.6e-8); 8 x 1024 took
+/// 14.1 us and takes 14.5, 16 x 2048 68 and 72. A weight as one fused v * log2(e)
+/// - k, k whole, saves that, but not 1 at the max: rows of one key are then off
+/// by 2e-8.
+template <>
+struct StatsQ<64> {
+    double l;
+    float m;
+};
+
+/// What a sum of weights against the max `from` is to be multiplied by to be
+/// one against the max `to` (finite, or the sum is NaN), no less.
+__device__ __forceinline__ double rebase(float from, float to) {
+    const double y = (static_cast<double>(from) - static_cast<double>(to)) * 1.4426950408889634074;
+    return exp2Poly(y < -1000.0 ? -1000.0 : y, kExp2C10);
+}
+
+/// exp2 of a score less a max, in the base of the head dim's scores.
+template <int D>
+__device__ __forceinline__ float weightQ(float v, float max) {
+    return __builtin_amdgcn_exp2f(D == 64 ? (v - max) * kLog2e : v - max);
 }
 
 /// 256 threads: global -> registers for the 128-key panel of K (its batch's
@@ -163,9 +200,9 @@ __device__ __forceinline__ void blockOfQ(int seq, int nr, int per, int64_t& b, i
 /// keys [k0, k0 + keys): D = K Q^T per 128-key panel, so each lane keeps a
 /// running max and sum(exp2(v - max)) of its query; the lane 32 away holds
 /// the other keys of the same query and the pair is combined at the end.
-/// Returns (max, sum) of query row `qrow` in base 2 (both half-waves agree).
+/// Returns those of query row `qrow` (both half-waves agree).
 template <int D, bool RAGGED>
-__device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
+__device__ __forceinline__ StatsQ<D> statsRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                               const float* __restrict__ bias, int seq, int sseq, float c2, int64_t b,
                                               int rb, int k0, int keys, _Float16* ldsQ, int64_t& qrow) {
     float* lbias = reinterpret_cast<float*>(ldsQ + 2 * kPanelHalvesQ<D>);  // this key range's bias
@@ -178,13 +215,14 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
     f16x8 xq[KS];                                 // B operand: this lane's query, KS x 16 head dims
 #pragma unroll
     for (int ks = 0; ks < KS; ++ks) xq[ks] = *reinterpret_cast<const f16x8*>(qr + ks * 16 + hl * 8);
-    for (int i = tid; i < keys; i += 256) lbias[i] = RAGGED && k0 + i >= sseq ? -INFINITY : biasLog2(bias[k0 + i]);
+    for (int i = tid; i < keys; i += 256) lbias[i] = RAGGED && k0 + i >= sseq ? -INFINITY : biasQ<D>(bias[k0 + i]);
     const _Float16* kb = K + b * (RAGGED ? sseq : seq) * D;
     u32x4v v[D / 16];
     loadPanelQ<D, RAGGED>(kb, k0, sseq, tid, v);
     storePanelQ<D>(ldsQ, tid, v);
     __syncthreads();
-    float m = -INFINITY, l = 0.0f;
+    float m = -INFINITY;
+    decltype(StatsQ<D>::l) l = 0;
     for (int p = 0; p < np; ++p) {
         if (p + 1 < np) loadPanelQ<D, RAGGED>(kb, k0 + (p + 1) * kPanelQ, sseq, tid, v);
         const _Float16* pk = ldsQ + (p & 1) * kPanelHalvesQ<D>;
@@ -217,62 +255,105 @@ __device__ __forceinline__ float2 statsRangeQ(const _Float16* __restrict__ Q, co
                 }
             }
         }
+        // The lane 32 away agrees on the max, so that f64 sums just add up.
+        if constexpr (D == 64) mb = fmaxf(mb, __shfl_xor(mb, 32, 64));
         // A panel whose scores are all -inf adds nothing: its exponentials
         // are taken against a finite stand-in for the -inf max.
         const float mn = fmaxf(m, mb);
         const float ms = finiteOr0(mn);
-        // Eight short sums: a quarter of one long one's rounding.
-        float sb[8];
+        if constexpr (D == 64) {
+            double sp = 0.0;
 #pragma unroll
-        for (int g = 0; g < 8; ++g) {
-            sb[g] = __builtin_amdgcn_exp2f(acc[g / 2][g % 2 * 8] - ms);
+            for (int i = 0; i < 4; ++i) {
 #pragma unroll
-            for (int r = 1; r < 8; ++r) sb[g] += __builtin_amdgcn_exp2f(acc[g / 2][g % 2 * 8 + r] - ms);
+                for (int r = 0; r < 16; r += 4) {
+                    float e[4];
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) e[q] = weightQ<D>(acc[i][r + q], ms);
+                    sp += static_cast<double>((e[0] + e[1]) + (e[2] + e[3]));
+                }
+            }
+            l = p > 0 ? l * rebase(m, ms) + sp : sp;
+        } else {
+            // Eight short sums: a quarter of one long one's rounding.
+            float sb[8];
+#pragma unroll
+            for (int g = 0; g < 8; ++g) {
+                sb[g] = weightQ<D>(acc[g / 2][g % 2 * 8], ms);
+#pragma unroll
+                for (int r = 1; r < 8; ++r) sb[g] += weightQ<D>(acc[g / 2][g % 2 * 8 + r], ms);
+            }
+            l = l * __builtin_amdgcn_exp2f(m - ms) +
+                (((sb[0] + sb[1]) + (sb[2] + sb[3])) + ((sb[4] + sb[5]) + (sb[6] + sb[7])));
         }
-        l = l * __builtin_amdgcn_exp2f(m - ms) +
-            (((sb[0] + sb[1]) + (sb[2] + sb[3])) + ((sb[4] + sb[5]) + (sb[6] + sb[7])));
         m = mn;
         if (p + 1 < np) storePanelQ<D>(ldsQ + ((p + 1) & 1) * kPanelHalvesQ<D>, tid, v);
         __syncthreads();
     }
-    const float mo = __shfl_xor(m, 32, 64);
-    const float lo = __shfl_xor(l, 32, 64);
-    const float mx = fmaxf(m, mo);
-    const float ms = finiteOr0(mx);
-    const float lt = l * __builtin_amdgcn_exp2f(m - ms) + lo * __builtin_amdgcn_exp2f(mo - ms);
-    return make_float2(mx, lt);
+    if constexpr (D == 64) {
+        StatsQ<D> st;
+        st.m = m;
+        st.l = l + __shfl_xor(l, 32, 64);
+        return st;
+    } else {
+        const float mo = __shfl_xor(m, 32, 64);
+        const float lo = __shfl_xor(l, 32, 64);
+        const float mx = fmaxf(m, mo);
+        const float ms = finiteOr0(mx);
+        return {mx, l * __builtin_amdgcn_exp2f(m - ms) + lo * __builtin_amdgcn_exp2f(mo - ms)};
+    }
 }
 
+/// Key ranges of a row that a lane merges.
+template <int D>
+constexpr int kRangesOfLaneQ = D == 64 ? kMaxRangesQ / 2 : kMaxRangesQ;
+
 /// Row statistics of the 16 rows this lane's pass-2 accumulators hold: lane
-/// l32 merges row r0 + l32's nr partials pp (base 2; those past nr repeat the
-/// first) into shift and scale, which the lanes then pass around. Pass 2
-/// writes exp2(v - shift) * scale, scale 1 / sum(exp2(v - shift)). The shift is
-/// the row's max, or 0 for a row whose max is in [0, 64]: that subtraction has
+/// l32 merges row r0 + l32's nr partials pp (those past nr repeat the first)
+/// into shift and scale, which the lanes then pass around; at head dim 64 the
+/// lane 32 away has half of them. Pass 2 writes exp(v - shift) * scale, scale 1
+/// / sum(exp(v - shift)), in the base of the scores. The shift is the row's
+/// max, or, at 128, 0 for a row whose max is in [0, 64]: that subtraction has
 /// no rounding and is left out, and what then underflows, v < -126, is below
 /// float's normal range after the scale too.
 /// A log-normalizer max + log2(sum) in one float as the shift would save the
 /// multiply, and cost 2^-24 of its magnitude in every value of the row.
 /// A row whose scores are all -inf keeps max -inf: exp2(-inf - -inf) writes
 /// NaN, as the reference does. Returns whether every row's shift is 0.
-__device__ __forceinline__ bool mergeStatsQ(const float2 (&pp)[kMaxRangesQ], int nr, float (&shift)[16],
+template <int D>
+__device__ __forceinline__ bool mergeStatsQ(const StatsQ<D> (&pp)[kRangesOfLaneQ<D>], int nr, float (&shift)[16],
                                             float (&scale)[16]) {
     const int hl = (threadIdx.x & 63) >> 5;
-    float m = pp[0].x;
+    float m = pp[0].m;
 #pragma unroll
-    for (int i = 1; i < kMaxRangesQ; ++i) m = fmaxf(m, pp[i].x);
-    const bool plain = m >= 0.0f && m <= 64.0f;
-    const float sh = plain ? 0.0f : m;
-    const float ms = finiteOr0(sh);
-    float lt = 0.0f;
+    for (int i = 1; i < kRangesOfLaneQ<D>; ++i) m = fmaxf(m, pp[i].m);
+    float sh, sc;
+    bool plain = false;
+    if constexpr (D == 64) {
+        sh = fmaxf(m, __shfl_xor(m, 32, 64));
+        const float ms = finiteOr0(sh);
+        double lt = 0.0;
 #pragma unroll
-    for (int i = 0; i < kMaxRangesQ; ++i) lt += i < nr ? pp[i].y * __builtin_amdgcn_exp2f(pp[i].x - ms) : 0.0f;
-    const float sc = 1.0f / lt;
+        for (int i = 0; i < kRangesOfLaneQ<D>; ++i) {
+            const double part = pp[i].l * rebase(pp[i].m, ms);
+            lt += hl * kRangesOfLaneQ<D> + i < nr ? part : 0.0;
+        }
+        sc = static_cast<float>(1.0 / (lt + __shfl_xor(lt, 32, 64)));
+    } else {
+        plain = m >= 0.0f && m <= 64.0f;
+        sh = plain ? 0.0f : m;
+        const float ms = finiteOr0(sh);
+        float lt = 0.0f;
+#pragma unroll
+        for (int i = 0; i < kMaxRangesQ; ++i) lt += i < nr ? pp[i].l * __builtin_amdgcn_exp2f(pp[i].m - ms) : 0.0f;
+        sc = 1.0f / lt;
+    }
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
         shift[r] = __shfl(sh, 8 * (r >> 2) + 4 * hl + (r & 3), 64);
         scale[r] = __shfl(sc, 8 * (r >> 2) + 4 * hl + (r & 3), 64);
     }
-    return __all(plain);
+    return D != 64 && __all(plain);
 }
 
 /// Pass 2 over keys [k0, k0 + keys) of this wave's 32 rows r0..r0+31 of
@@ -291,7 +372,7 @@ template <int D, bool RAGGED, bool QUADS>
 __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                             const float* __restrict__ bias, float* __restrict__ S, int seq,
                                             int sseq, float c2, int64_t b, int rb, int64_t r0, int k0, int keys,
-                                            const float2* __restrict__ part, int nr, _Float16* ldsQ) {
+                                            const StatsQ<D>* __restrict__ part, int nr, _Float16* ldsQ) {
     const int ld = RAGGED ? sseq : seq;           // S row length
     const int i0 = static_cast<int>(r0 - b * seq);   // first row within the batch
     const int tid = threadIdx.x;
@@ -314,14 +395,17 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
     for (int r = 0; r < 16; ++r) {
         soff[r] = static_cast<uint32_t>(((8 * (r >> 2) + 4 * hl + (r & 3)) * ld + lk) * sizeof(float));
     }
-    float2 pp[kMaxRangesQ];
+    StatsQ<D> pp[kRangesOfLaneQ<D>];
 #pragma unroll
-    for (int i = 0; i < kMaxRangesQ; ++i) pp[i] = part[(r0 + l32) * nr + (i < nr ? i : 0)];
+    for (int i = 0; i < kRangesOfLaneQ<D>; ++i) {
+        const int range = (D == 64 ? hl * kRangesOfLaneQ<D> : 0) + i;
+        pp[i] = part[(r0 + l32) * nr + (range < nr ? range : 0)];
+    }
     u32x4v v[D / 16];
     int at = static_cast<int>(b) % np;
     loadPanelQ<D, RAGGED>(kb, k0 + at * kPanelQ, ld, tid, v);
     float shift[16], scale[16];
-    const bool plain = mergeStatsQ(pp, nr, shift, scale);
+    const bool plain = mergeStatsQ<D>(pp, nr, shift, scale);
     storePanelQ<D, QUADS>(ldsQ, tid, v);
     __syncthreads();
     for (int p = 0; p < np; ++p) {
@@ -345,7 +429,7 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
         }
         float bj[4];
 #pragma unroll
-        for (int j = 0; j < 4; ++j) bj[j] = biasLog2(bias[RAGGED ? min(kc + lk + j * jk, ld - 1) : kc + lk + j * jk]);
+        for (int j = 0; j < 4; ++j) bj[j] = biasQ<D>(bias[RAGGED ? min(kc + lk + j * jk, ld - 1) : kc + lk + j * jk]);
         char* sb = reinterpret_cast<char*>(S + (b * ld + i0) * static_cast<int64_t>(ld) + kc);
         auto store = [&](auto value) {
 #pragma unroll
@@ -367,7 +451,7 @@ __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, cons
         if (plain) {
             store([&](float v, int r) { return __builtin_amdgcn_exp2f(v) * scale[r]; });
         } else {
-            store([&](float v, int r) { return __builtin_amdgcn_exp2f(v - shift[r]) * scale[r]; });
+            store([&](float v, int r) { return weightQ<D>(v, shift[r]) * scale[r]; });
         }
         if (p + 1 < np) storePanelQ<D, QUADS>(ldsQ + ((p + 1) & 1) * kPanelHalvesQ<D>, tid, v);
         __syncthreads();
@@ -378,14 +462,14 @@ template <int D, bool RAGGED>
 __global__ __launch_bounds__(256, 2) void scoreStatsQ(const _Float16* __restrict__ Q,
                                                       const _Float16* __restrict__ K,
                                                       const float* __restrict__ bias,
-                                                      float2* __restrict__ part, int seq, int sseq, int nr, int per,
+                                                      StatsQ<D>* __restrict__ part, int seq, int sseq, int nr, int per,
                                                       float c2) {
     extern __shared__ __align__(16) _Float16 ldsQ[];
     int64_t b;
     int rb, kr, k0, keys;
     blockOfQ(seq, nr, per, b, rb, kr, k0, keys);
     int64_t qrow;
-    const float2 st = statsRangeQ<D, RAGGED>(Q, K, bias, seq, sseq, c2, b, rb, k0, keys, ldsQ, qrow);
+    const StatsQ<D> st = statsRangeQ<D, RAGGED>(Q, K, bias, seq, sseq, c2, b, rb, k0, keys, ldsQ, qrow);
     if (((threadIdx.x & 63) >> 5) == 0) part[qrow * nr + kr] = st;
 }
 
@@ -393,7 +477,7 @@ template <int D, bool RAGGED, bool QUADS>
 __global__ __launch_bounds__(256, 2) void scoreStoreQ(const _Float16* __restrict__ Q,
                                                       const _Float16* __restrict__ K,
                                                       const float* __restrict__ bias,
-                                                      const float2* __restrict__ part, float* __restrict__ S,
+                                                      const StatsQ<D>* __restrict__ part, float* __restrict__ S,
                                                       int seq, int sseq, int nr, int per,
                                                       float c2) {
     extern __shared__ __align__(16) _Float16 ldsQ[];
@@ -463,16 +547,16 @@ int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragge
     const size_t ldsStats = kLdsStoreQ<D> + static_cast<size_t>(per) * sizeof(float);
     const int nr = rangesQ(p, most);
     const dim3 grid(static_cast<unsigned>(p->batch * (p->seq / kPanelQ) * nr));
-    // Both passes work in base 2: v2 = acc * (log2(e) / div) + bias * log2(e),
-    // exp(v - max) = exp2(v2 - max2).
-    const float c2 = static_cast<float>(1.4426950408889634 / p->div);
+    // At head dim 128 both passes work in base 2: v2 = acc * (log2(e) / div) +
+    // bias * log2(e), exp(v - max) = exp2(v2 - max2).
+    const float c2 = static_cast<float>((D == 64 ? 1.0 : 1.4426950408889634) / p->div);
     hipLaunchKernelGGL(stats, grid, dim3(256), ldsStats, st, static_cast<const _Float16*>(p->q),
                        static_cast<const _Float16*>(p->k), static_cast<const float*>(p->bias),
-                       static_cast<float2*>(p->scratch), static_cast<int>(p->seq),
+                       static_cast<StatsQ<D>*>(p->scratch), static_cast<int>(p->seq),
                        static_cast<int>(sseq), nr, per, c2);
     hipLaunchKernelGGL(store, grid, dim3(256), kLdsStoreQ<D>, st,
                        static_cast<const _Float16*>(p->q), static_cast<const _Float16*>(p->k),
-                       static_cast<const float*>(p->bias), static_cast<const float2*>(p->scratch),
+                       static_cast<const float*>(p->bias), static_cast<const StatsQ<D>*>(p->scratch),
                        static_cast<float*>(p->s), static_cast<int>(p->seq),
                        static_cast<int>(sseq), nr, per, c2);
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
@@ -481,8 +565,8 @@ int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragge
 /// `div` is held to where 1 / div times log2(e) is a normal float.
 /// Head dim 64 takes it from 512 keys, and more rows than that: with fewer it
 /// gains nothing (3 x 256: 7.9 against 7.4 us, 1 x 512: 8.0 and 7.7, 2 x 512:
-/// 7.8 and 8.3) and with fewer keys its error is the larger (16 x 128: 1.30e-7
-/// against 1.24e-7; 2 x 512: 1.38e-7 and 1.40e-7, 8 x 1024: 1.42e-7 and 1.44e-7).
+/// 8.1 and 8.3). Its error is the other form's (2 x 512: 1.39e-7 and 1.39e-7,
+/// 8 x 1024: 1.44e-7 and 1.45e-7, 1 x 8192: 1.67e-7 and 1.66e-7).
 bool twoPassApplies(const mlkd_score_softmax* p) {
     const double size = p->div < 0 ? -p->div : p->div;
     if (!(size >= 1e-30 && size <= 1e30)) return false;
@@ -496,7 +580,7 @@ bool twoPassApplies(const mlkd_score_softmax* p) {
 /// Row statistics partials of nr key ranges: one (max, sum) pair per row and
 /// range.
 int64_t statsBytes(const mlkd_score_softmax* p, int nr) {
-    return p->batch * p->seq * nr * static_cast<int64_t>(sizeof(float2));
+    return p->batch * p->seq * nr * static_cast<int64_t>(p->dim == 64 ? sizeof(StatsQ<64>) : sizeof(StatsQ<128>));
 }
 
 template <typename T>

@@ -24,6 +24,7 @@
 #include <math.h>
 #include <stdint.h>
 
+#include "exp2_poly.h"
 #include "mlk_device_math.h"
 #include "runtime_abi.h"
 
@@ -278,8 +279,8 @@ __global__ __launch_bounds__(256) void softmaxWaveRowPipelined(const float* x, f
     }
 }
 
-/// 2^f on |f| <= 1/2 by Chebyshev interpolation at N nodes: relative error
-/// 2.5e-9 (N = 7), 5.5e-11 (N = 8), 1.9e-14 (N = 10).
+/// exp2Poly's coefficients with fewer terms: relative error 2.5e-9 (7),
+/// 5.5e-11 (8).
 constexpr double kExp2C7[7] = {1.0,
                                0.6931472067028326,
                                0.24022650922288757,
@@ -290,24 +291,6 @@ constexpr double kExp2C7[7] = {1.0,
 constexpr double kExp2C8[8] = {0.9999999999595618,     0.6931471805568324,    0.24022651213498092,
                                0.055504109063258665,   0.009618025613318018,  0.0013333478473685175,
                                0.00015469729214122798, 1.5303700711425663e-05};
-constexpr double kExp2C10[10] = {1.0000000000000135,    0.6931471805599462,     0.2402265069564034,
-                                 0.05550410866465166,   0.00961812919393429,    0.0013333558200796013,
-                                 0.0001540343375126647, 1.5252672924257465e-05, 1.3259645241948732e-06,
-                                 1.020590550210069e-07};
-
-/// 2^y (times the coefficients' common factor) for y in [-1000, 1000]; NaN
-/// stays NaN. y + 1.5 * 2^52 leaves rint(y) in the low word, from where it is
-/// added into the exponent field.
-template <int N>
-__device__ __forceinline__ double exp2Poly(double y, const double (&c)[N]) {
-    const double t = y + 0x1.8p52;
-    const double f = y - (t - 0x1.8p52);
-    double p = c[N - 1];
-#pragma unroll
-    for (int i = N - 2; i >= 0; --i) p = __builtin_fma(p, f, c[i]);
-    return __hiloint2double(__double2hiint(p) + (__double2loint(t) << 20), __double2loint(p));
-}
-
 template <typename T>
 struct WideRow;
 template <>

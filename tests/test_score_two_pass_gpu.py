@@ -88,6 +88,31 @@ def test_no_live_key_and_nan(hip, b, s, d):
     assert np.isnan(got[0, 7]).all() and np.isnan(got).sum() == s
 
 
+# A row's weights add up to 1 but for the rounding of 1 / sum, at most u, evenly
+# spread (u / sqrt(3) rms), and of the weights, at most 2 u of each, by chance (2 u
+# sqrt(sum of p^2)); sums in f32 are off by twice that.
+@pytest.mark.parametrize("b,s", [(16, 512), (3, 640), (8, 1024), (2, 2048), (1, 8192)])
+def test_row_sums_at_dim_64(hip, b, s):
+    q, k, bias = operands(b, s, 64)
+    p = np.asarray(built(hip, b, s, 64).run({0: q.reshape(-1), 1: k.reshape(-1), 2: bias})[3], np.float64).reshape(-1, s)
+    off = p.sum(axis=1) - 1
+    assert np.sqrt((off ** 2).mean()) <= U * (1 / np.sqrt(3) + 2 * np.sqrt((p ** 2).sum(axis=1).mean()))
+
+
+# Masks past float's range in base 2 keep their order; +inf makes its row NaN.
+def test_bias_at_the_ends_of_the_range_at_dim_64(hip):
+    b, s = 2, 512
+    q, k, bias = operands(b, s, 64)
+    art = built(hip, b, s, 64)
+    bias[:] = np.finfo(np.float32).min
+    bias[[3, 130, 511]] = -2.5e38
+    got = np.asarray(art.run({0: q.reshape(-1), 1: k.reshape(-1), 2: bias})[3]).reshape(-1, s)
+    assert (got[:, [3, 130, 511]] == np.float32(1 / 3)).all()
+    assert not np.delete(got, [3, 130, 511], 1).any()
+    bias[7] = np.inf
+    assert np.isnan(np.asarray(art.run({0: q.reshape(-1), 1: k.reshape(-1), 2: bias})[3])).all()
+
+
 class _At:
     def __init__(self, n, skip):
         self.buf, self.skip, self.n = DeviceBuffer.from_array(np.zeros(n + 8, np.float32), "f32"), skip, n
