@@ -95,9 +95,9 @@ int mlkd_rt_malloc_spare(void** p, size_t bytes, void* stream) {
     hipStreamCaptureStatus status = hipStreamCaptureStatusNone;
     if (hipStreamIsCapturing(static_cast<hipStream_t>(stream), &status) != hipSuccess) {
         (void)hipGetLastError();
-        return MLKD_RT_ALLOC;
+        return -1;
     }
-    if (status != hipStreamCaptureStatusNone) return MLKD_RT_ALLOC;
+    if (status != hipStreamCaptureStatusNone) return -1;
     hipStreamCaptureMode mode = hipStreamCaptureModeRelaxed;
     if (hipThreadExchangeStreamCaptureMode(&mode) != hipSuccess) {
         (void)hipGetLastError();

@@ -26,8 +26,9 @@ int mlkd_rt_device_arch(int dev, char* buf, size_t cap);
 int mlkd_rt_device_info(int dev, int* cu_count, int64_t* max_grid_x, int* max_block,
                         int64_t* global_mem);
 int mlkd_rt_malloc(void** p, size_t bytes);
-/// mlkd_rt_malloc for memory the caller can do without: fails while `stream`
-/// is being captured and leaves a capture elsewhere in the process alone.
+/// mlkd_rt_malloc for memory the caller can do without: -1, and nothing tried,
+/// while `stream` is being captured; leaves a capture elsewhere in the process
+/// alone.
 int mlkd_rt_malloc_spare(void** p, size_t bytes, void* stream);
 int mlkd_rt_free(void* p);
 /// Page-locked host memory (hipHostMalloc): copies between it and the device

@@ -268,6 +268,7 @@ HipLoadedKernel::RunScratch& HipLoadedKernel::scratchFor(void* stream) const {
     rs->tempElems.assign(km_.buffers.size(), 0);
     rs->step.assign(plan_.steps.size(), nullptr);
     rs->stepBytes.assign(plan_.steps.size(), 0);
+    rs->stepWait.resize(plan_.steps.size());
     scratchByStream_.emplace_back(stream, std::move(rs));
     return *scratchByStream_.back().second;
 }
@@ -281,19 +282,21 @@ int64_t HipLoadedKernel::stepScratch(RunScratch& rs, size_t si, int64_t need, in
     std::lock_guard<std::mutex> g(scratchLock_);
     void*& p = rs.step[si];
     int64_t& bytes = rs.stepBytes[si];
-    if (bytes < (need > 0 ? need : want)) {
-        void* block = nullptr;
-        int64_t size = 0;
-        if (want > need && mlkd_rt_malloc_spare(&block, static_cast<size_t>(want), stream) == 0) {
-            size = want;
-        } else if (need > 0 && mlkd_rt_malloc(&block, static_cast<size_t>(need)) == 0) {
-            size = need;
-        }
-        if (size > 0) {
-            if (p != nullptr) rs.outgrown.push_back(p);
-            p = block;
-            bytes = size;
-        }
+    RunScratch::Wait& wait = rs.stepWait[si];
+    void* block = nullptr;
+    int64_t size = 0;
+    if (bytes < want && wait.left > 0) {
+        --wait.left;
+    } else if (bytes < want) {
+        const int rc = mlkd_rt_malloc_spare(&block, static_cast<size_t>(want), stream);
+        if (rc == 0) size = want;
+        else if (rc > 0 && need > 0) wait.left = wait.last = std::min(2 * wait.last + 1, 1 << 16);
+    }
+    if (size == 0 && bytes < need && mlkd_rt_malloc(&block, static_cast<size_t>(need)) == 0) size = need;
+    if (size > 0) {
+        if (p != nullptr) rs.outgrown.push_back(p);
+        p = block;
+        bytes = size;
     }
     *ptr = p;
     return bytes;

@@ -114,15 +114,24 @@ private:
         void* status{nullptr};
         std::vector<void*> step;
         std::vector<int64_t> stepBytes;
+        /// Of a step that makes do with a smaller block: runs left until it
+        /// asks for the larger again, and how many it waited the last time.
+        struct Wait {
+            int32_t left{0}, last{0};
+        };
+        std::vector<Wait> stepWait;
         std::vector<void*> outgrown;   // smaller blocks of `step`: a captured graph may still use them
     };
     RunScratch& scratchFor(void* stream) const;  // caller holds scratchLock_
     static void freeScratch(RunScratch& rs);
-    /// Bytes of rs.step[si] (at *ptr), allocated on first use: `want` where the step can
-    /// do without it and they can be had (not while `stream` is captured),
-    /// otherwise `need`; less than that when the allocation fails. A GEMM's
-    /// `want` varies with the alignment of its operands (copies of A, of B or
-    /// of both), so a step outgrows at most two blocks.
+    /// Bytes of rs.step[si] (at *ptr), allocated on first use: `want` where the
+    /// step can do without it and they can be had (not while `stream` is
+    /// captured), otherwise `need`; less than that when the allocation fails. A
+    /// step with less than `want` asks for it again: where `need` is 0 on every
+    /// run, otherwise after 1, 3, 7, ... runs, since memory that is short stays so
+    /// for a while and a refusal takes its time. A GEMM's `want` varies with the
+    /// alignment of its operands (copies of A, of B or of both), so a step
+    /// outgrows at most two blocks.
     int64_t stepScratch(RunScratch& rs, size_t si, int64_t need, int64_t want, void* stream, void** ptr) const;
     /// Offsets of a run's scratch in `arena`; refuses what does not fit or
     /// needs a host read-back.

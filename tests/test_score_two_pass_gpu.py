@@ -160,9 +160,11 @@ def test_allocation_free_entry_without_room(hip):
 
 
 class _Capture:
-    """Captures what is enqueued on a new stream into a HIP graph."""
+    """Captures what is enqueued on a new stream into a HIP graph (mode 0:
+    nothing may allocate meanwhile, 2: relaxed)."""
 
-    def __init__(self):
+    def __init__(self, mode=0):
+        self.mode = mode
         with open("/proc/self/maps") as f:
             path = next(line.split()[-1] for line in f if "libamdhip64" in line)
         self.hip, self.stream, self.graph, self.exec = ctypes.CDLL(path), *(ctypes.c_void_p() for _ in range(3))
@@ -172,7 +174,7 @@ class _Capture:
         assert getattr(self.hip, name)(*args) == 0, name
 
     def __enter__(self):
-        self("hipStreamBeginCapture", self.stream, 0)
+        self("hipStreamBeginCapture", self.stream, self.mode)
         return self.stream.value
 
     def __exit__(self, *exc):
@@ -214,4 +216,25 @@ def test_first_run_under_capture(hip, case):
                 check(got, q, k, bias)
             else:
                 assert (np.abs(got.reshape(128, 128) - a @ b) <= 2 * 4099 * 2.0 ** -53 * (np.abs(a) @ np.abs(b))).all()
+    cap.close()
+
+
+# A stream's first run under a relaxed capture gets the scratch it needs, for two
+# key ranges, and no workspace for eight; a later run asks for that again, and
+# the graph keeps its own.
+def test_workspace_after_a_captured_first_run(hip):
+    q, k, bias = operands(1, 2048, 128)
+    art, bufs = built(hip, 1, 2048, 128), device(q, k, bias)
+    out, eager, fresh = (DeviceBuffer(2048 * 2048, "f32") for _ in range(3))
+    built(hip, 1, 2048, 128).run_device({**bufs, 3: fresh})
+    cap = _Capture(mode=2)
+    with cap as stream:
+        art.run_device({**bufs, 3: out}, stream=stream, sync=False)
+    for _ in range(3):
+        cap.replay()
+        check(out.to_numpy(), q, k, bias)
+        art.run_device({**bufs, 3: eager}, stream=cap.stream.value, sync=False)
+        cap("hipStreamSynchronize", cap.stream)
+        assert np.array_equal(eager.to_numpy(), fresh.to_numpy())
+    assert not np.array_equal(out.to_numpy(), fresh.to_numpy())     # two ranges add up in another order
     cap.close()
