@@ -2253,6 +2253,8 @@ bool raggedShape(const mlkd_gemm* p) {
     // 200x2000x2000: 29 against 40 us).
     if (f16 && (p->m + kRM - 1) / kRM * ((p->n + kRN - 1) / kRN) < 64 && p->k >= 256) return false;
     if (f32 && pm / kFM * (pn / kFN) <= 128 && p->k >= 128) return false;
+    // A grid holds fewer than 2^32 threads (2^23 tiles: a C of 137 GB).
+    if (f32 && pm / kFM * (pn / kFN) >= (int64_t{1} << 32) / 512) return false;
     const double work = static_cast<double>(p->m) * static_cast<double>(p->n) * static_cast<double>(p->k);
     return 2.0 * work >= static_cast<double>(int64_t{1} << 30) ||
            static_cast<double>(pm) * static_cast<double>(pn) * static_cast<double>(pk) <= 8.0 * work;
