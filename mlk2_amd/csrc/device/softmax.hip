@@ -279,18 +279,6 @@ __global__ __launch_bounds__(256) void softmaxWaveRowPipelined(const float* x, f
     }
 }
 
-/// exp2Poly's coefficients with fewer terms: relative error 2.5e-9 (7),
-/// 5.5e-11 (8).
-constexpr double kExp2C7[7] = {1.0,
-                               0.6931472067028326,
-                               0.24022650922288757,
-                               0.05550327226670302,
-                               0.009618056678524643,
-                               0.0013400428177615916,
-                               0.00015461444698568514};
-constexpr double kExp2C8[8] = {0.9999999999595618,     0.6931471805568324,    0.24022651213498092,
-                               0.055504109063258665,   0.009618025613318018,  0.0013333478473685175,
-                               0.00015469729214122798, 1.5303700711425663e-05};
 template <typename T>
 struct WideRow;
 template <>
@@ -298,8 +286,6 @@ struct WideRow<float> {
     static constexpr int V = 4;
     static constexpr float kMostMax = 1e6f;
     using Vec = f32x4;
-    static constexpr const auto& cSum = kExp2C7;
-    static constexpr const auto& cOut = kExp2C8;
     static __device__ __forceinline__ float narrow(double v) { return static_cast<float>(v); }
 };
 template <>
@@ -307,8 +293,6 @@ struct WideRow<_Float16> {
     static constexpr int V = 8;
     static constexpr float kMostMax = 60000.0f;
     using Vec = _Float16 __attribute__((ext_vector_type(8)));
-    static constexpr const auto& cSum = kExp2C10;
-    static constexpr const auto& cOut = kExp2C10;
     /// One rounding of v >= 0: to the nearest f32, made round-to-odd (one
     /// step down if that was up, the last bit set if inexact), then to f16.
     static __device__ __forceinline__ _Float16 narrow(double v) {
@@ -348,12 +332,15 @@ __device__ __forceinline__ void softmaxOddRow(const T* x, T* y, int cols, float 
 /// per row, CH 16-byte pieces of it in each lane's registers in T, so the row
 /// is read once and written once. Pieces start at the row's first 16-byte
 /// boundary; the up to V - 1 elements before it and after the last whole
-/// piece go one to a lane of the first wave. 2^y takes 12-15 f64 instructions
+/// piece go one to a lane of the first wave. 2^y takes 15 f64 instructions
 /// (which issue at the f32 rate here), so it is computed twice, for the sum
-/// and for the output, rather than held in two registers per element.
-/// 1000 x 30001 f32 takes 57 us, 4.2 TB/s (softmaxBlockRow, which reads the row
-/// three times and calls exp twice: 219 us; a copy of the same bytes: 45 us),
-/// 8192 x 4096 f16 54 us (160 us). The f64 work, about 30 us of each, and the
+/// and for the output, rather than held in two registers per element. With
+/// polynomials of 7 terms for the sum and 8 for the output (2.5e-9 and 5.5e-11
+/// off) results were not the exact ones rounded once, 6% of them in rows of two
+/// values; those of 10 (1.9e-14) take 1000 x 30001 f32 from 54.5 to 55.7 us,
+/// 4.3 TB/s (softmaxBlockRow, which reads the row three times and calls exp
+/// twice: 219 us; a copy of the same bytes: 45 us). 8192 x 4096 f16 takes 54 us
+/// (160 us). The f64 work, about 30 us of each, and the
 /// memory traffic overlap only between the two to four rows a CU holds.
 /// Summing against a reference of the row's first pieces, so that a piece's
 /// terms are computed under the loads of the next, took 72 us; walking rows
@@ -364,7 +351,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softma
     using R = WideRow<T>;
     using Vec = typename R::Vec;
     constexpr int V = R::V;
-    constexpr int NOut = sizeof(R::cOut) / sizeof(double);
+    constexpr int NOut = sizeof(kExp2C10) / sizeof(double);
     __shared__ float smax[W];
     __shared__ double ssum[W];
     const int lane = threadIdx.x & 63;
@@ -426,14 +413,14 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softma
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             v[c][i] = v[c][i] < lo ? lo : v[c][i];
-            s += exp2Poly(exponent(v[c][i]), R::cSum);
+            s += exp2Poly(exponent(v[c][i]), kExp2C10);
         }
         // The terms are recomputed below, not kept.
         asm volatile("" : "+v"(v[c]), "+v"(s));
     }
     if (w == 0) {
         one = one < lo ? lo : one;
-        s += exp2Poly(exponent(one), R::cSum);
+        s += exp2Poly(exponent(one), kExp2C10);
     }
     s = acrossWaves<W, false>(waveSum(s), ssum);
     // s >= 1 or NaN, as in normalizeRow. A NaN row's outputs are all NaN (set
@@ -443,7 +430,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softma
     double co[NOut];
 #pragma unroll
     for (int i = 0; i < NOut; ++i) {   // uniform over the row's waves: scalar registers
-        const double k = R::cOut[i] * inv;
+        const double k = kExp2C10[i] * inv;
         co[i] = __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(k)),
                                  __builtin_amdgcn_readfirstlane(__double2loint(k)));
     }

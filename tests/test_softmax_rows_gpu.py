@@ -3,9 +3,8 @@ past 8192 columns, f16 rows; softmaxWaveRowScalar past 4096 columns), at the
 edges of their ranges, against the oracle's f64 softmax.
 
 Bounds: f32 results of f64 arithmetic round once, so each is within 1 ULP of
-the oracle's value (2^-23 of it; 2.5e-9 of that is the polynomial's), or
-2^-149 of a subnormal one; f16 results are the oracle's rounded once (the
-polynomial's 1.9e-14 moves none here). The f32 arithmetic of the shorter rows
+the oracle's value (2^-23 of it), or 2^-149 of a subnormal one; f16 results are
+the oracle's rounded once (the polynomial's 1.9e-14 moves none here). The f32 arithmetic of the shorter rows
 is held to the class's 1e-6."""
 import numpy as np
 import pytest
@@ -92,6 +91,23 @@ def test_rows_of_large_values(hip, n, skip, in_place):
     yb = xb if in_place else _At(np.zeros_like(x), "f32", skip)
     art.run_device({0: xb, 1: yb})
     check(yb.values(), x, "f32")
+
+
+# Of a row of two values every term but one has the same polynomial error: the
+# results are the exact ones rounded once. 1.9e-14 of the term, as much of the sum
+# and 2e-14 of its additions, against half an ULP of 2^-25 or more, are below
+# 2^-18 of that half. With terms off by 2.5e-9 some 6% of them round elsewhere.
+@pytest.mark.parametrize("n", [8200, 20000, 65535])
+def test_rows_of_two_values(hip, n):
+    c = np.random.default_rng(n).uniform(0.0, 12.0, 200).astype(np.float32)
+    x = np.repeat(-c[:, None], n, axis=1)
+    x[:, 0] = 0.0
+    got = np.asarray(hip.build(fx.softmax_call_module(*x.shape, "f32")).run({0: x.reshape(-1)})[1]).reshape(x.shape)
+    assert (got[:, 1:] == got[:, 1:2]).all()
+    e = np.exp(-c.astype(np.float64))
+    for have, ref in ((got[:, 0], 1 / (1 + (n - 1) * e)), (got[:, 1], e / (1 + (n - 1) * e))):
+        half = np.spacing(ref.astype(np.float32)).astype(np.float64) / 2
+        assert (np.abs(have - ref) <= half * (1 + 2.0 ** -18)).all()
 
 
 class _At:
