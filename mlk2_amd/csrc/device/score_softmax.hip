@@ -562,7 +562,9 @@ int launchQ(const mlkd_score_softmax* p, int most, hipStream_t st, int64_t ragge
     return hipGetLastError() == hipSuccess ? 0 : MLKD_RT_LAUNCH;
 }
 
-/// `div` is held to where 1 / div times log2(e) is a normal float.
+/// `div` is held to where 1 / div times log2(e) is a normal float, the grid to
+/// the fewer than 2^32 threads that HIP takes (2^24 batches of a few keys are
+/// 4 GiB of Q).
 /// Head dim 64 takes it from 512 keys, and more rows than that: with fewer it
 /// gains nothing (3 x 256: 7.9 against 7.4 us, 1 x 512: 8.0 and 7.7, 2 x 512:
 /// 8.1 and 8.3). Its error is the other form's (2 x 512: 1.39e-7 and 1.39e-7,
@@ -574,7 +576,7 @@ bool twoPassApplies(const mlkd_score_softmax* p) {
            (p->dim == 64 || p->dim == 128) && p->seq % kPanelQ == 0 && p->seq > 0 && p->seq <= kMaxSeqQ &&
            (p->dim == 128 || (p->seq >= 512 && p->batch * p->seq > 512)) &&
            (reinterpret_cast<uintptr_t>(p->q) & 15u) == 0 && (reinterpret_cast<uintptr_t>(p->k) & 15u) == 0 &&
-           p->batch * (p->seq / kPanelQ) * 8 <= 0x7FFFFFFF;
+           p->batch <= (int64_t{1} << 32) / 256 && p->batch * (p->seq / kPanelQ) * rangesQ(p) < (int64_t{1} << 32) / 256;
 }
 
 /// Row statistics partials of nr key ranges: one (max, sum) pair per row and
