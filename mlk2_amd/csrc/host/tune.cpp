@@ -329,16 +329,11 @@ std::string launchCoverage(const KernelModule& km, const Step& st, int64_t eleme
             // f32 rows of at most 8192 (cols % 4 == 0) run the wave path:
             // form 5 (the default) two rows per wave, form 1 a fixed grid of
             // 2048 waves, the other forms a row per wave, at most 8192
-            // workgroups; anything else a workgroup per row.
+            // workgroups. The other rows have one form each, and a step
+            // without a choice is not reported.
             instances = st.rows;
-            auto dt = [&](uint32_t b) { return km.buffers[b].dtype; };
-            const bool wave = dt(st.x) == Dtype::F32 && dt(st.y) == Dtype::F32 && st.cols % 4 == 0 && st.cols <= 8192;
             const int v = st.variant >= 0 ? st.variant : 5;
-            if (!wave) {
-                workgroups = std::min<int64_t>(std::max<int64_t>(st.rows, 1), 65536);
-                perGroup = 1;
-                form = "a workgroup per row, grid-stride";
-            } else if (v == 5) {
+            if (v == 5) {
                 workgroups = std::min<int64_t>(std::max<int64_t>(((st.rows + 1) / 2 + 3) / 4, 1), 8192);
                 perGroup = 8;
                 form = "two adjacent rows per wave, grid-stride";
