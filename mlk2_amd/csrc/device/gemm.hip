@@ -1564,7 +1564,9 @@ constexpr size_t kLdsRagged = static_cast<size_t>(kDmaStages) * kRStage * sizeof
 /// a CU, bounded as dma8sTile<ACC, true> is. A K step takes 0.31 us for each
 /// tile on a CU, one or two: its LDS traffic (32 KiB of reads, half of them
 /// transposed, 16 KiB of direct loads; 256 x 128 tiles of 8 waves, a quarter
-/// less to load, are no faster). 2000 x 1000 x 3000 takes 24.5 us, with C += A
+/// less to load, are no faster). A text of its own, since the schedule is fenced
+/// MFMA by MFMA, and 16 a step with 8 fragments to read have other places for
+/// the reads, loads and barrier than 32 with 12. 2000 x 1000 x 3000 takes 24.5 us, with C += A
 /// B 27.9 us (zero-padded copies of A, B and C around 256 x 256 tiles: 44.4
 /// and 59.7 us), 2000^3 25 us (58 us), 1000 x 600 x 1000 10.4 us (28 us).
 template <bool ACC>

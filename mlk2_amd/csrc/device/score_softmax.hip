@@ -5,11 +5,13 @@
 //
 // The output write (4 * batch * seq^2 bytes) bounds the class; the scores are
 // a GEMM with K = dim on v_mfma_f32_32x32x16_f16. Forms, best first:
-//   * two-pass, query-stationary (dim 128, or 64 from 512 keys, seq % 128 == 0,
-//     seq <= 8192): a statistics pass and a recompute-and-write pass (scoreStatsQ /
-//     scoreStoreQ), rows' partial statistics in artifact scratch;
-//   * scores, then the softmax kernel in place over S (any shape, f16);
-//   * a scalar f64 path for other dtypes.
+//   * two-pass, query-stationary (dim 128 at any length, dim 64 from 512 keys at
+//     multiples of 128; up to 8192 keys): a statistics pass and a
+//     recompute-and-write pass (scoreStatsQ / scoreStoreQ), rows' partial
+//     statistics in artifact scratch;
+//   * scores, then the softmax kernel in place over S (f16, multiples of 128
+//     keys, head dims that are multiples of 16);
+//   * a scalar f64 path for other dtypes and shapes.
 #include <hip/hip_runtime.h>
 
 #include <cstdio>
@@ -72,12 +74,13 @@ __global__ __launch_bounds__(256) void scoresF16(const _Float16* __restrict__ Q,
 typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 
 // Query-stationary form of the two passes (head dim D 64 or 128, seq a
-// multiple of 128). A wave owns 32 query rows and holds their Q fragments in
+// multiple of 128, or at 128 bounded). A wave owns 32 query rows and holds their Q fragments in
 // registers for the whole kernel; a workgroup of 4 waves (128 rows) streams one
 // of NR ranges of the batch's keys through LDS in 128-key panels, double
 // buffered, the next panel's global loads in flight during the current panel's
-// MFMAs. At most 73 KiB of LDS and 256 registers per lane let two workgroups
-// share a CU. Scores by 64 x 128 tiles and a softmax over S in place read S
+// MFMAs. Two workgroups share a CU: at most 256 registers per lane, and 68 KiB
+// of LDS at D 128 (36 at 64), to which pass 1 adds 4 bytes for each key of its
+// range; past 24 panels that leaves room for one. Scores by 64 x 128 tiles and a softmax over S in place read S
 // back and each K element once per 64 rows: at D 64, 8 x 1024 took 23.5 us
 // and takes 14.5, 16 x 2048 165 and 72.
 //   Pass 1 (scoreStatsQ) computes D = K Q^T per panel, so each lane holds 64
@@ -86,14 +89,15 @@ typedef uint32_t u32x4v __attribute__((ext_vector_type(4)));
 //   keys of the same query, and the pair is combined once at the end into
 //   scratch[row][key range].
 //   Pass 2 (scoreStoreQ) computes D = Q K^T per panel and writes
-//   softmax of the panel at once: each 32-lane half-wave stores
-//   one 128-byte line, while the other workgroup on the CU computes.
+//   softmax of the panel at once, 512 bytes of each of two rows to a store
+//   (storeRangeQ), while the other workgroup on the CU computes.
 // At D 128 both passes work in base 2 with log2(e) folded into 1/div and the
 // bias, so a score costs one fused multiply-add and one v_exp_f32; at D 64 in
 // base e, with f64 sums (StatsQ<64>). 16 x 2048 x 128: pass
-// 1 takes 29 us, bound by its v_exp_f32 (13 us) and MFMAs (7 us), which the
-// two waves of a SIMD overlap in part (panels of 64 keys and four workgroups a
-// CU: no faster); pass 2 takes 45-48 us, bound by its 256 MiB of stores.
+// 1 takes 29-34 us by the clock, bound by its v_exp_f32 (13 us) and MFMAs (7
+// us), which the two waves of a SIMD overlap in part (panels of 64 keys and four
+// workgroups a CU: no faster); pass 2 takes 47-50 us, bound by its 256 MiB of
+// stores. The pair: 77-87 us from box to box.
 constexpr int kPanelQ = 128;                   // keys per streamed panel
 constexpr int kMaxRangesQ = 8;                 // key ranges per 128-row block
 constexpr float kLog2e = 1.44269504088896340736f;
@@ -182,8 +186,9 @@ __device__ __forceinline__ void storePanelQ(_Float16* dst, int tid, const u32x4v
 /// Workgroup coordinates: batch, 128-row block, key range of nr, and the
 /// range's first key and length: `per` keys, the last range what is left. A
 /// batch's workgroups are contiguous within one XCD's share of the grid, a row
-/// block's side by side (ranges as the slow dimension: 16 x 2048 x 128 90.7
-/// against 77 us). Grids of no multiple of 8 in grid order: 9 x 640 x 128 13.0
+/// block's side by side (ranges as the slow dimension: 16 x 2048 x 64 73.5 against
+/// 70.2 us, 8 x 1024 x 64 16.0 against 14.5; 16 x 2048 x 128 79.4 against 76.8 on
+/// one box, 83 against 85 on another). Grids of no multiple of 8 in grid order: 9 x 640 x 128 13.0
 /// against 12.1 us, 13 x 1280 x 64 29.6 against 28.3.
 __device__ __forceinline__ void blockOfQ(int seq, int nr, int per, int64_t& b, int& rb, int& kr, int& k0, int& keys) {
     const int panels = seq / kPanelQ;
@@ -366,8 +371,9 @@ __device__ __forceinline__ bool mergeStatsQ(const StatsQ<D> (&pp)[kRangesOfLaneQ
 /// writes 128.
 /// Batches start at different panels: row blocks in step would write the same
 /// few columns of rows a power of two apart, which share memory channels (16 x
-/// 2048 x 128, both passes: 90.6 -> 77 us; x 64: 81 -> 67). Within a batch they
-/// stay in step, for K in the L2 (each row block apart: 84 and 74 us).
+/// 2048 x 128, both passes: 89.1 -> 76.8 us on one box, 90.7 -> 85.4 on another;
+/// x 64: 84 -> 70 on both). Within a batch they stay in step, for K in the L2
+/// (each row block apart: 84 us where this takes 77).
 template <int D, bool RAGGED, bool QUADS>
 __device__ __forceinline__ void storeRangeQ(const _Float16* __restrict__ Q, const _Float16* __restrict__ K,
                                             const float* __restrict__ bias, float* __restrict__ S, int seq,
