@@ -337,10 +337,13 @@ __device__ __forceinline__ void softmaxOddRow(const T* x, T* y, int cols, float 
 /// and for the output, rather than held in two registers per element. With
 /// polynomials of 7 terms for the sum and 8 for the output (2.5e-9 and 5.5e-11
 /// off) results were not the exact ones rounded once, 6% of them in rows of two
-/// values; those of 10 (1.9e-14) take 1000 x 30001 f32 from 54.5 to 55.7 us,
+/// values; those of 10 (1.9e-14) take 1000 x 30001 f32 from 54.5 to 56.1 us,
 /// 4.3 TB/s (softmaxBlockRow, which reads the row three times and calls exp
 /// twice: 219 us; a copy of the same bytes: 45 us). 8192 x 4096 f16 takes 54 us
-/// (160 us). The f64 work, about 30 us of each, and the
+/// (160 us). Pieces past the row are skipped, each by a uniform branch: 4000 x
+/// 8196 f32 59.5 us (computed for nothing 71.7), 800 x 40000 84.8-88.6 (94), f16
+/// 2000 x 20000 73 (79), but 512 x 65536, which has none, 72-75 (70); by twos or
+/// fours no faster. The f64 work, about 30 us of each, and the
 /// memory traffic overlap only between the two to four rows a CU holds.
 /// Summing against a reference of the row's first pieces, so that a piece's
 /// terms are computed under the loads of the next, took 72 us; walking rows
@@ -410,6 +413,7 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softma
     double s = 0.0;
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
+        if (c * (W * 64) >= whole) continue;   // past the row in every lane
 #pragma unroll
         for (int i = 0; i < V; ++i) {
             v[c][i] = v[c][i] < lo ? lo : v[c][i];
@@ -442,10 +446,11 @@ __global__ __launch_bounds__(W == 1 ? 256 : 64 * W, CH >= 8 ? 4 : 8) void softma
     if (single >= 0) yr[single] = result(one);
 #pragma unroll
     for (int c = 0; c < CH; ++c) {
+        const int first = c * (W * 64);
+        if (first >= whole) continue;
         Vec o;
 #pragma unroll
         for (int i = 0; i < V; ++i) o[i] = result(v[c][i]);
-        const int first = c * (W * 64);
         char* base = reinterpret_cast<char*>(yr + head) + first * 16;
         if (piece < whole - first) {
             __builtin_nontemporal_store(o, reinterpret_cast<Vec*>(base + static_cast<uint32_t>(piece) * 16u));
